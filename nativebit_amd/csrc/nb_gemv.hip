@@ -20,8 +20,9 @@
 //   DPP, then across groups through LDS after one barrier.
 // * gemv_generic_kernel: any shape, bits 1..8, M <= 16.  One workgroup per
 //   output row, lanes stride over k and read each field from the byte
-//   stream.  Used for ragged shapes and as an independent statement of the
-//   arithmetic.
+//   stream.  Used for ragged shapes (K not a multiple of 128, other formats)
+//   and as an independent statement of the arithmetic; several fp32 rows of
+//   the standard formats run nb_gemm_rows.hip.
 //
 // Arithmetic for both: with fp32 x the exact fp32 codebook value, with bf16 x
 // the codebook value rounded to bf16 (the reference's bf16 semantics,
@@ -33,6 +34,7 @@
 // kernel in nb_gemv_mfma.hip before either kernel here is considered.
 #include "nb_device.h"
 #include "nb_internal.h"
+#include "nb_lookup.h"
 #include "nb_stream_common.h"
 
 #include <algorithm>
@@ -119,47 +121,6 @@ __global__ __launch_bounds__(kThreads) void fill_zero_kernel(void* y, int dtype,
 // ---------------------------------------------------------------------------
 // fast M == 1 kernel
 // ---------------------------------------------------------------------------
-// (a & mask) | b in one VALU op, the mask in a scalar register (the disjoint
-// `or` would otherwise become an add after a separate and).
-__device__ __forceinline__ uint32_t and_or_s(uint32_t a, uint32_t mask, uint32_t b) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(mask), "v"(b));
-    return r;
-}
-
-// LDS byte address of codebook entry (field j) in the lane's table:
-// `base` | field << POS.  POS = 8 for a lane's entry-major copy (the wave's
-// table holds entry e of lane l at byte 256 e + 4 l, so every lookup of a
-// wave hits a bank of its own); POS = 2 for the block's own NE entries where
-// they landed in LDS.  `base` has zeros in the field's bits.  The field is
-// shifted straight to bit POS and merged with the base: two VALU ops a
-// weight (the fields of a 3-bit slice that straddle a dword take a funnel
-// shift).
-template <int BITS, int J, int POS>
-__device__ __forceinline__ uint32_t entry_offset(const uint32_t (&d)[BITS], uint32_t base) {
-    constexpr int bit = J * BITS;
-    constexpr int w = bit >> 5;
-    constexpr int off = bit & 31;
-    constexpr uint32_t kMask = ((1u << BITS) - 1u) << POS;
-    uint32_t v;
-    if constexpr (off + BITS > 32) {
-        v = __builtin_amdgcn_alignbit(d[w + 1], d[w], off - POS);
-    } else if constexpr (off >= POS) {
-        v = d[w] >> (off - POS);
-    } else {
-        v = d[w] << (POS - off);
-    }
-    return and_or_s(v, kMask, base);
-}
-
-typedef __attribute__((address_space(3))) const float lds_f32;
-
-template <int BITS, int POS, int J0, int... Js>
-__device__ __forceinline__ void lookup8(const uint32_t (&d)[BITS], uint32_t base, float (&w)[8],
-                                        std::integer_sequence<int, Js...>) {
-    ((w[Js] = *(lds_f32*)(uintptr_t)entry_offset<BITS, J0 + Js, POS>(d, base)), ...);
-}
-
 // sum_j cb[field j] * x[j] over the 32 weights of a slice.  Lookups are
 // issued eight at a time into registers before the FMAs so that the LDS
 // latency overlaps, and two accumulators shorten the FMA chain.
@@ -539,6 +500,10 @@ int launch_gemv(const GemvArgs& a, hipStream_t stream) {
                            plan.depth);
         return check_launch("nb_gemv (fast)");
     }
+    // several fp32 rows, or one that the kernel above does not take (K an odd
+    // multiple of 128, or over 8192): 10-13 times faster than a workgroup per
+    // row at every measured size from 513 x 384 up
+    if (gemm_rows_f32_eligible(a)) return launch_gemm_rows_f32(a, stream);
     int64_t grid = a.N;
     if (grid > (int64_t)cus * 16) grid = (int64_t)cus * 16;
     hipLaunchKernelGGL(gemv_generic_kernel, dim3((int)grid), dim3(kThreads), 0, stream, a);
