@@ -191,6 +191,12 @@ int launch_rope_kv_rows(const float* qkv, float* k_cache, float* v_cache, const 
 int launch_attention_rows(const float* q, const float* k_cache, const float* v_cache, int pos0,
                           int T, void* out, int out_dtype, int n_head, int D, int ctx,
                           hipStream_t stream);
+// The same on fp32 MFMAs for head dims 64 and 128 over `batch` sequences
+// (nb_attention_mfma.hip): whether it takes the operands, and its launch.
+bool attention_mfma_eligible(const float* q, const float* k, const float* v, int D, int ctx);
+int launch_attention_mfma(const float* q, const float* k, const float* v, int pos0, int T,
+                          void* out, int out_dtype, int batch, int n_head, int D, int ctx,
+                          hipStream_t stream);
 int attention_rows_max_head_dim();
 
 // Persistent decode (nb_decode_persistent.hip); arguments validated.

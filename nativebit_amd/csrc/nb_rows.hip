@@ -302,6 +302,13 @@ int launch_rope_kv_rows(const float* qkv, float* k_cache, float* v_cache, const 
 int launch_attention_rows(const float* q, const float* k_cache, const float* v_cache, int pos0,
                           int T, void* out, int out_dtype, int n_head, int D, int ctx,
                           hipStream_t stream) {
+    // fp32 MFMAs where the layout allows 16-byte loads; up to 32 positions at
+    // head dim 128 the vector kernel below is as fast or faster (16 queries
+    // from position 0: 8.0 us against 8.9; 64: 9.3 against 9.0)
+    if (attention_mfma_eligible(q, k_cache, v_cache, D, ctx) && (D < 128 || pos0 + T > 32)) {
+        return launch_attention_mfma(q, k_cache, v_cache, pos0, T, out, out_dtype, 1, n_head, D,
+                                     ctx, stream);
+    }
     hipLaunchKernelGGL(attention_rows_kernel, dim3(n_head, (T + kQB - 1) / kQB),
                        dim3(kAttThreads), 0, stream, q, k_cache, v_cache, pos0, T, out,
                        out_dtype, n_head, D, ctx);
