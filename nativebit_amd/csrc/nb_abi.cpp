@@ -926,7 +926,7 @@ extern "C" int nb_gemm_prefill_f32(const float* x, int64_t ldx, const uint8_t* p
                     (long long)need);
     }
     if (dev_st) return dev_st;
-    return launch_prefill_f32(x, ldx, packed, codebook, y, ldy, M, N, K, workspace, ws_bytes,
+    return launch_prefill_f32(x, ldx, packed, codebook, y, ldy, M, N, K, workspace,
                               static_cast<hipStream_t>(stream));
 }
 

@@ -6,7 +6,7 @@
 // materialises W on every call (inference/triton_kernel.py:258-275; in bf16,
 // inference/eval_ppl.py:149-174).  Here a 512-thread workgroup owns a BN x
 // BM tile of Y^T (BN = 256 or 128 outputs x BM = 256, 128 or 64 tokens,
-// chosen per launch by grid occupancy) and walks K in steps of 64:
+// chosen per launch by estimated time) and walks K in steps of 64:
 //
 //   * the X slice (BM tokens x 64 bf16) arrives by global_load_lds_dwordx4
 //     (eight rows per instruction), 16-byte chunk c of row r in LDS slot
@@ -30,6 +30,8 @@
 //     tiles of one or two token blocks rather than of all of them.
 // Weights are the codebook entries rounded to bf16 (RNE), as the bf16 path;
 // accumulation is fp32.
+#include <math.h>
+
 #include <algorithm>
 #include <type_traits>
 
@@ -107,7 +109,6 @@ struct Prefill2Args {
     int M, N, K;
     int ksplit;   // K ranges per output tile (1: the whole of K)
     float* part;  // ksplit > 1: fp32 partial products [ksplit][M][N], else null
-    int accumulate;  // fp32 y only: y += result instead of y = result
 };
 
 // Tile of the calling workgroup.  Workgroups are dealt to the 8 XCDs in
@@ -120,10 +121,10 @@ struct Prefill2Args {
 struct TileOf {
     int n0, m0;       // first output and first token of the tile
     int ks;           // K range of this workgroup
-    int s0, nsteps;   // its K steps: [s0, s0 + nsteps) of the K / 64
+    int s0, nsteps;   // its K steps: [s0, s0 + nsteps) of the K / STEPK
 };
 
-template <int BM, int BN>
+template <int BM, int BN, int STEPK>
 __device__ __forceinline__ TileOf tile_of(const Prefill2Args& a) {
     const int nn = (a.N + BN - 1) / BN;
     const int ntiles = nn * ((a.M + BM - 1) / BM);
@@ -134,8 +135,8 @@ __device__ __forceinline__ TileOf tile_of(const Prefill2Args& a) {
     const int tile = v - t.ks * ntiles;
     t.n0 = (tile % nn) * BN;
     t.m0 = (tile / nn) * BM;
-    t.s0 = (int)((int64_t)t.ks * (a.K / kBK) / a.ksplit);
-    t.nsteps = (int)((int64_t)(t.ks + 1) * (a.K / kBK) / a.ksplit) - t.s0;
+    t.s0 = (int)((int64_t)t.ks * (a.K / STEPK) / a.ksplit);
+    t.nsteps = (int)((int64_t)(t.ks + 1) * (a.K / STEPK) / a.ksplit) - t.s0;
     return t;
 }
 
@@ -175,14 +176,12 @@ __device__ __forceinline__ void store_tile(const Prefill2Args& a, const f32x4_t 
                 }
             } else {
                 float* yp = static_cast<float*>(yb) + (int64_t)m * ldy + n;
-                const bool acc_y = !partial && a.accumulate;
                 if (n + 3 < a.N && (reinterpret_cast<uintptr_t>(yp) & 15) == 0) {
-                    *reinterpret_cast<f32x4_t*>(yp) =
-                        acc_y ? *reinterpret_cast<const f32x4_t*>(yp) + v : v;
+                    *reinterpret_cast<f32x4_t*>(yp) = v;
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (n + e < a.N) yp[e] = acc_y ? yp[e] + v[e] : v[e];
+                        if (n + e < a.N) yp[e] = v[e];
                 }
             }
         }
@@ -199,7 +198,19 @@ struct WRegs {
     u32x4_t c0, c1;
 };
 
-template <int BM, int BN, int WAVES>
+// kSplit: fp32 activations against the exact fp32 weights as three bf16
+// products, x = hi + lo and W = hi + lo: hi.hi + hi.lo + lo.hi.  A step is 32
+// of K instead of 64, an LDS row its 32 hi parts (chunks 0-3) and its 32 lo
+// parts (chunks 4-7); x arrives already split, in that order (split_bf16_
+// kernel).  Of the two threads of a W row one dequantizes the hi parts
+// (entries rounded to bf16), the other the lo parts (what that rounding left,
+// rounded to bf16).  The fragments of a step then feed three MFMAs instead of
+// two, so this form reads less LDS per MFMA than the bf16 one.  Measured
+// against three passes of the bf16 kernel that added to y (and a residual
+// codebook made per call): 7680 x 2560 at M = 128 / 500 / 2048 37 / 84 / 236 us
+// (72 / 129 / 286), 2560 x 6912 40 / 73 / 245 us (78 / 145 / 313), the same
+// 4.3e-6 from fp64.
+template <int BM, int BN, int WAVES, bool kSplit>
 __global__ __launch_bounds__(64 * WAVES) void prefill2_kernel(Prefill2Args a) {
     constexpr int kThreads = 64 * WAVES;
     constexpr int WGM = WAVES >= 16 ? 4 : 2;  // waves along the tokens
@@ -216,10 +227,12 @@ __global__ __launch_bounds__(64 * WAVES) void prefill2_kernel(Prefill2Args a) {
     constexpr int H = 2 / TPR;           // 32-weight halves per thread
     constexpr bool kAllDeq = kThreads <= 2 * BN;
     static_assert(TPR == 1 || TPR == 2, "one or two threads per W row");
+    static_assert(!kSplit || TPR == 2, "one thread for the hi parts, one for the lo parts");
+    constexpr int kStepK = kSplit ? kBK / 2 : kBK;
     using WR = WRegs<H>;
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const TileOf t = tile_of<BM, BN>(a);
+    const TileOf t = tile_of<BM, BN, kStepK>(a);
     const int n0 = t.n0, m0 = t.m0, ks = t.ks, s0 = t.s0, nsteps = t.nsteps;
     const int bpr = a.K / 128;
     const uint32_t base = lds_addr(smem);
@@ -243,11 +256,13 @@ __global__ __launch_bounds__(64 * WAVES) void prefill2_kernel(Prefill2Args a) {
     const bool deq = kAllDeq || tid < 2 * BN;
     auto load_w = [&](int step, WR& w) {
         if (!deq) return;
-        const int64_t blk = (int64_t)gn * bpr + ((s0 + step) >> 1);
+        constexpr int kStepsLog = kSplit ? 2 : 1;   // steps a block
+        const int64_t blk = (int64_t)gn * bpr + ((s0 + step) >> kStepsLog);
+        const int in_blk = (s0 + step) & ((1 << kStepsLog) - 1);
 #pragma unroll
         for (int h = 0; h < H; ++h) {
             const uint32_t* ip = reinterpret_cast<const uint32_t*>(
-                a.packed + blk * 48 + ((s0 + step) & 1) * 24 + (h0 + h) * 12);
+                a.packed + blk * 48 + (kSplit ? in_blk * 12 : in_blk * 24 + (h0 + h) * 12));
             w.d[h].x = ip[0];
             w.d[h].y = ip[1];
             w.d[h].z = ip[2];
@@ -258,10 +273,22 @@ __global__ __launch_bounds__(64 * WAVES) void prefill2_kernel(Prefill2Args a) {
     };
     auto store_w = [&](int stage, const WR& w) {
         if (!deq) return;
-        const uint32_t q0 = pack_bf16x2(__uint_as_float(w.c0.x), __uint_as_float(w.c0.y));
-        const uint32_t q1 = pack_bf16x2(__uint_as_float(w.c0.z), __uint_as_float(w.c0.w));
-        const uint32_t q2 = pack_bf16x2(__uint_as_float(w.c1.x), __uint_as_float(w.c1.y));
-        const uint32_t q3 = pack_bf16x2(__uint_as_float(w.c1.z), __uint_as_float(w.c1.w));
+        uint32_t q0 = pack_bf16x2(__uint_as_float(w.c0.x), __uint_as_float(w.c0.y));
+        uint32_t q1 = pack_bf16x2(__uint_as_float(w.c0.z), __uint_as_float(w.c0.w));
+        uint32_t q2 = pack_bf16x2(__uint_as_float(w.c1.x), __uint_as_float(w.c1.y));
+        uint32_t q3 = pack_bf16x2(__uint_as_float(w.c1.z), __uint_as_float(w.c1.w));
+        if constexpr (kSplit) {
+            // entry - bf16(entry), exact in fp32
+            auto rest = [](uint32_t q, uint32_t a0, uint32_t a1) {
+                return pack_bf16x2(__uint_as_float(a0) - __uint_as_float(q << 16),
+                                   __uint_as_float(a1) - __uint_as_float(q & 0xffff0000u));
+            };
+            const bool lo = h0 != 0;
+            q0 = lo ? rest(q0, w.c0.x, w.c0.y) : q0;
+            q1 = lo ? rest(q1, w.c0.z, w.c0.w) : q1;
+            q2 = lo ? rest(q2, w.c1.x, w.c1.y) : q2;
+            q3 = lo ? rest(q3, w.c1.z, w.c1.w) : q3;
+        }
         const uint32_t lo0 = __builtin_amdgcn_perm(q1, q0, 0x06040200u);
         const uint32_t hi0 = __builtin_amdgcn_perm(q1, q0, 0x07050301u);
         const uint32_t lo1 = __builtin_amdgcn_perm(q3, q2, 0x06040200u);
@@ -316,15 +343,17 @@ __global__ __launch_bounds__(64 * WAVES) void prefill2_kernel(Prefill2Args a) {
         if (step + 1 < nsteps) load_x(step + 1, cur ^ 1);
         const unsigned char* xt = smem + cur * kStage;
         const unsigned char* wt = xt + kXBytes;
-        auto mfma_k32 = [&](int ks) {  // 32 of the step's 64 K
-            const int c = ks * 4 + fq;
-            u32x4_t av[TI], bv[TJ];
+        auto read_w = [&](int c, u32x4_t (&av)[TI]) {
 #pragma unroll
             for (int i = 0; i < TI; ++i)
-                av[i] = *reinterpret_cast<const u32x4_t*>(wt + swz(wn * WN + i * 16 + fr, c));
+                av[i] = *reinterpret_cast<const u32x4_t*>(wt + swz(wn * WN + i * 16 + fr, c + fq));
+        };
+        auto read_x = [&](int c, u32x4_t (&bv)[TJ]) {
 #pragma unroll
             for (int j = 0; j < TJ; ++j)
-                bv[j] = *reinterpret_cast<const u32x4_t*>(xt + swz(wm * WM + j * 16 + fr, c));
+                bv[j] = *reinterpret_cast<const u32x4_t*>(xt + swz(wm * WM + j * 16 + fr, c + fq));
+        };
+        auto mfma_all = [&](const u32x4_t (&av)[TI], const u32x4_t (&bv)[TJ]) {
 #pragma unroll
             for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -333,9 +362,28 @@ __global__ __launch_bounds__(64 * WAVES) void prefill2_kernel(Prefill2Args a) {
                         __builtin_bit_cast(bf16x8_t, av[i]), __builtin_bit_cast(bf16x8_t, bv[j]),
                         acc[i][j], 0, 0, 0);
         };
-        mfma_k32(0);
-        if (step + 1 < nsteps) store_w(cur ^ 1, next);
-        mfma_k32(1);
+        if constexpr (kSplit) {
+            u32x4_t wv[TI], xv[TJ];
+            read_w(0, wv);
+            read_x(0, xv);
+            mfma_all(wv, xv);
+            u32x4_t wlo[TI];
+            read_w(4, wlo);
+            if (step + 1 < nsteps) store_w(cur ^ 1, next);
+            mfma_all(wlo, xv);
+            read_x(4, xv);
+            mfma_all(wv, xv);
+        } else {
+            // 32 of the step's 64 K, then the other 32
+            u32x4_t av[TI], bv[TJ];
+            read_w(0, av);
+            read_x(0, bv);
+            mfma_all(av, bv);
+            if (step + 1 < nsteps) store_w(cur ^ 1, next);
+            read_w(4, av);
+            read_x(4, bv);
+            mfma_all(av, bv);
+        }
         // the next X slice (direct-to-LDS, not tracked by the compiler) must
         // be in LDS before the barrier; the W loads of step + 2, issued
         // before it, have had the whole step to arrive
@@ -352,12 +400,11 @@ __global__ __launch_bounds__(64 * WAVES) void prefill2_kernel(Prefill2Args a) {
 
 // y[m][n] = sum over k ranges s = 0, 1, ... of part[s][m][n] (in that
 // order, so the result does not depend on which workgroup finished first),
-// converted to y's dtype (added to fp32 y with accumulate).  Four
-// consecutive outputs per thread where the rows allow it.
+// converted to y's dtype.  Four consecutive outputs per thread where the
+// rows allow it.
 __global__ __launch_bounds__(256) void prefill_reduce_kernel(const float* __restrict__ part,
                                                              int S, int M, int N, void* y,
-                                                             int y_dtype, int64_t ldy,
-                                                             int accumulate) {
+                                                             int y_dtype, int64_t ldy) {
     const int64_t plane = (int64_t)M * N;
     // four outputs a thread where every row starts on a 4-output boundary
     // of both part and y (rows of 4k outputs, bases aligned for the vector
@@ -378,8 +425,7 @@ __global__ __launch_bounds__(256) void prefill_reduce_kernel(const float* __rest
                 p.y = (uint32_t)f32_to_bf16_rne(v.z) | ((uint32_t)f32_to_bf16_rne(v.w) << 16);
                 *reinterpret_cast<u32x2_t*>(static_cast<bf16_bits*>(y) + m * ldy + n) = p;
             } else {
-                f32x4_t* yp = reinterpret_cast<f32x4_t*>(static_cast<float*>(y) + m * ldy + n);
-                *yp = accumulate ? *yp + v : v;
+                *reinterpret_cast<f32x4_t*>(static_cast<float*>(y) + m * ldy + n) = v;
             }
         } else {
             const int64_t m = i / N, n = i - m * N;
@@ -388,8 +434,7 @@ __global__ __launch_bounds__(256) void prefill_reduce_kernel(const float* __rest
             if (y_dtype == NB_BF16) {
                 static_cast<bf16_bits*>(y)[m * ldy + n] = f32_to_bf16_rne(v);
             } else {
-                float* yp = static_cast<float*>(y) + m * ldy + n;
-                *yp = accumulate ? *yp + v : v;
+                static_cast<float*>(y)[m * ldy + n] = v;
             }
         }
     }
@@ -399,82 +444,142 @@ struct PrefillPlan {
     int BM, BN, S;
 };
 
-// The tile (BM tokens x BN outputs) and the number of K ranges per tile.
-// One launch over all of K: the largest tile (fewest workgroups, least
-// redundant traffic) whose grid still gives about 0.6 workgroups per CU.
-// Where only the smallest tile (64 x 128) is left -- few tokens or a narrow
-// layer, where every workgroup walks all of K with little work per step --
-// and a split is allowed, the largest tile that reaches that grid when
-// repeated over S <= 8 K ranges of at least 8 steps each, preferring fp32
-// partial products (written, then read once by the reduction) of at most
-// twice the packed weight's bytes, else four times.  Measured on MI355X
-// over the four 2.2B layer shapes: M = 128 layer 140 -> 86 us, M = 512
-// 191 -> 156-162 us (down 75 -> 44-45 us); splitting tiles that already
-// fill the grid was slower.  A tile that reaches 0.6 per CU but leaves more
-// than a tenth of the CUs idle gives way to 256 x 256 over S K ranges when
-// K is long (below).
+// What a tile costs, in microseconds: `step[c - 1]` a K step of 64 with c of
+// its workgroups resident on a CU (as many as its LDS allows), `start` from a
+// workgroup's launch to its first step and from its last to its end.  Fitted
+// to about 1900 measured plans on MI355X (six layer shapes from 1024 x 4096 to
+// 13824 x 2560, M = 32 .. 2048, every tile, S = 1 .. 16; mean error 6 %).
+struct TileCost {
+    int BM, BN, resident;
+    float start, step[3];
+};
+constexpr TileCost kBf16Tiles[] = {{256, 256, 1, 5.9f, {1.71f}},
+                                   {256, 128, 1, 3.4f, {1.09f}},
+                                   {128, 128, 2, 3.3f, {0.74f, 1.15f}},
+                                   {64, 128, 3, 2.7f, {0.57f, 0.91f, 1.42f}}};
+// three products (two steps of 32 per 64 of K; they spill at 256 x 256)
+constexpr TileCost kF32Tiles[] = {{256, 128, 1, 0.4f, {2.55f}},
+                                  {128, 128, 2, 1.2f, {1.76f, 3.34f}},
+                                  {64, 128, 3, 1.2f, {1.34f, 2.00f, 3.03f}}};
+constexpr int kMinSplitSteps = 4;
+
+inline int64_t grid_of(int M, int N, int bm, int bn) {
+    return (int64_t)((N + bn - 1) / bn) * ((M + bm - 1) / bm);
+}
+
+// Estimated time of S K ranges per tile: the busiest CU takes
+// ceil(workgroups / CUs) of them, `resident` at a time; S > 1 adds the
+// reduction launch (r0) and the partial products' write and read (rb a MB).
+float plan_time(const TileCost& c, int S, int M, int N, int K, int64_t cus, float r0, float rb) {
+    const int64_t per = (grid_of(M, N, c.BM, c.BN) * S + cus - 1) / cus;
+    const int64_t conc = std::min<int64_t>(per, c.resident);
+    const float rounds = (float)((per + conc - 1) / conc);
+    const float t = rounds * (c.start + (float)((K / kBK + S - 1) / S) * c.step[conc - 1]);
+    return S > 1 ? t + r0 + rb * 4e-6f * (float)S * (float)M * (float)N : t;
+}
+
+// The plan of least estimated time.  bf16: K ranges only where the unsplit
+// grid of 128 x 128 tiles leaves more than 0.4 of the CUs without a
+// workgroup -- few tokens or a narrow layer --, at most 8 of them with
+// partial products of at most four times the packed weight's bytes; and,
+// where a tile reaches that grid but leaves a tenth of the CUs idle over a
+// long K, 256 x 256 over K ranges of at least 32 steps (down at M = 2048: 160
+// tiles of 256 x 128 126-135 us, 3 x 80 of 256 x 256 92-98 us).
+// Against fixed thresholds for the tile too: 2560 x 2560 at M = 32 / 64 23.5 /
+// 24.0 -> 11.7 / 13.3 us, 1024 x 4096 35 -> 12 us, 5000 x 1024 at M = 300 22 ->
+// 14.6 us, 2560 x 6912 at M = 700 55 -> 47 us; the sizes that the thresholds
+// were tuned on keep their plans or ones as fast.
 PrefillPlan prefill_plan(int M, int N, int K, bool allow_split) {
     const int64_t cus = device_cu_count();
-    const int64_t want = cus * 3 / 5;
     const int nsteps = K / kBK;
-    const int64_t wbytes = (int64_t)N * K / 128 * 80;
-    auto groups = [&](int bm, int bn) {
-        return (int64_t)((N + bn - 1) / bn) * ((M + bm - 1) / bm);
-    };
-    const int tiles[4][2] = {{256, 256}, {256, 128}, {128, 128}, {64, 128}};
-    for (int t = 0; t < 3; ++t) {
-        const int64_t g = groups(tiles[t][0], tiles[t][1]);
-        if (g < want) continue;
-        // A long K on a grid that still leaves a tenth of the CUs idle: the
-        // 256 x 256 tile over S K ranges of at least 32 steps, where that
-        // gives more workgroups (down at M = 2048: 160 tiles of 256 x 128
-        // 126-135 us, 3 x 80 of 256 x 256 92-98 us; o, whose K ranges would
-        // be 13 steps, stays at 51-54 us unsplit).
-        if (allow_split && M >= 256 && g * 10 < cus * 9) {
-            const int64_t g2 = groups(256, 256);
-            const int S = (int)std::min<int64_t>(cus / g2, nsteps / 32);
-            if (S >= 2 && g2 * S > g) return {256, 256, S};
+    const int64_t limit = 4 * ((int64_t)N * K / 128 * 80);
+    PrefillPlan best = {64, 128, 1};
+    float best_t = INFINITY;
+    auto offer = [&](const TileCost& c, int S) {
+        const float t = plan_time(c, S, M, N, K, cus, 5.5f, 0.30f);
+        if (t < best_t) {
+            best_t = t;
+            best = {c.BM, c.BN, S};
         }
-        return {tiles[t][0], tiles[t][1], 1};
+    };
+    for (const TileCost& c : kBf16Tiles) offer(c, 1);
+    if (!allow_split) return best;
+    int64_t full = 0;   // the grid of the largest tile that fills 0.6 of the CUs
+    for (int i = 0; i < 3 && !full; ++i) {
+        const int64_t g = grid_of(M, N, kBf16Tiles[i].BM, kBf16Tiles[i].BN);
+        if (g >= cus * 3 / 5) full = g;
     }
-    if (allow_split) {
-        for (int64_t mult = 2; mult <= 4; mult += 2) {
-            for (int t = 0; t < 4; ++t) {
-                const int bm = tiles[t][0], bn = tiles[t][1];
-                if (bm > std::max(64, M)) continue;   // mostly empty token rows
-                const int64_t g = groups(bm, bn);
-                int S = (int)std::min<int64_t>({cus / g, 8, nsteps / 8});
-                while (S > 1 && (int64_t)S * M * N * 4 > mult * wbytes) --S;
-                if (S > 1 && g * S >= want) return {bm, bn, S};
+    if (full) {
+        if (M >= 256 && full * 10 < cus * 9) {
+            const int64_t g = grid_of(M, N, 256, 256);
+            const int S = (int)std::min<int64_t>(cus / g, nsteps / 32);
+            if (S >= 2 && g * S > full) offer(kBf16Tiles[0], S);
+        }
+        return best;
+    }
+    best_t *= 1.1f;   // (the estimates' error: split where it costs about the same)
+    for (const TileCost& c : kBf16Tiles) {
+        for (int S = 2; S <= 8 && nsteps / S >= kMinSplitSteps; ++S) {
+            if ((int64_t)S * M * N * 4 <= limit) offer(c, S);
+        }
+    }
+    return best;
+}
+
+// fp32 activations: any number of K ranges up to 16 whose partial products
+// fit `limit` bytes (2560 x 2560 at M = 64 56 -> 22 us).
+PrefillPlan prefill_f32_plan(int M, int N, int K, int64_t limit) {
+    const int64_t cus = device_cu_count();
+    PrefillPlan best = {64, 128, 1};
+    float best_t = INFINITY;
+    for (const TileCost& c : kF32Tiles) {
+        for (int S = 1; S <= 16; ++S) {
+            if (S > 1 && (K / kBK / S < kMinSplitSteps || (int64_t)S * M * N * 4 > limit)) break;
+            const float t = plan_time(c, S, M, N, K, cus, 8.7f, 0.43f);
+            if (t < best_t) {
+                best_t = t;
+                best = {c.BM, c.BN, S};
             }
         }
     }
-    return {64, 128, 1};
+    return best;
 }
 
-// x (M rows, stride ldx, fp32) -> hi = bf16(x), lo = bf16(x - hi), rows of
-// K (contiguous).  x - hi is exact in fp32, so hi + lo is x to 2^-18.
+// x (M rows, stride ldx, fp32) -> for every 32 columns of a row their hi =
+// bf16(x), then their lo = bf16(x - hi): rows of 2K.  x - hi is exact in
+// fp32, so hi + lo is x to 2^-18.  A thread takes eight columns (16-byte
+// loads where kVec says that the rows allow them, 16-byte stores).
+template <bool kVec>
 __global__ __launch_bounds__(256) void split_bf16_kernel(const float* __restrict__ x, int64_t ldx,
-                                                         bf16_bits* __restrict__ hi,
-                                                         bf16_bits* __restrict__ lo, int M, int K) {
-    const int64_t total = (int64_t)M * K;
+                                                         bf16_bits* __restrict__ out, int M, int K) {
+    const int k8 = K / 8;
+    const int64_t total = (int64_t)M * k8;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total;
          i += (int64_t)gridDim.x * 256) {
-        const int64_t m = i / K, k = i - m * K;
-        const float v = x[m * ldx + k];
-        const bf16_bits h = f32_to_bf16_rne(v);
-        hi[i] = h;
-        lo[i] = f32_to_bf16_rne(v - bf16_to_f32(h));
-    }
-}
-
-// The residual codebook: cb_lo = cb - bf16(cb) (exact in fp32).
-__global__ __launch_bounds__(256) void cb_residual_kernel(const float* __restrict__ cb,
-                                                          float* __restrict__ cb_lo, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * 256) {
-        const float v = cb[i];
-        cb_lo[i] = v - bf16_to_f32(f32_to_bf16_rne(v));
+        const int64_t m = i / k8;
+        const int k = 8 * (int)(i - m * k8);
+        const float* p = x + m * ldx + k;
+        float v[8];
+        if (kVec) {
+            const f32x4_t a = reinterpret_cast<const f32x4_t*>(p)[0];
+            const f32x4_t b = reinterpret_cast<const f32x4_t*>(p)[1];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = a[e], v[4 + e] = b[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = p[e];
+        }
+        u32x4_t hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const bf16_bits h0 = f32_to_bf16_rne(v[2 * e]), h1 = f32_to_bf16_rne(v[2 * e + 1]);
+            hi[e] = h0 | ((uint32_t)h1 << 16);
+            lo[e] = f32_to_bf16_rne(v[2 * e] - bf16_to_f32(h0)) |
+                    ((uint32_t)f32_to_bf16_rne(v[2 * e + 1] - bf16_to_f32(h1)) << 16);
+        }
+        bf16_bits* o = out + m * 2 * K + (k / 32) * 64 + k % 32;
+        *reinterpret_cast<u32x4_t*>(o) = hi;
+        *reinterpret_cast<u32x4_t*>(o + 32) = lo;
     }
 }
 
@@ -482,75 +587,27 @@ inline int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
 }  // namespace
 
-int64_t prefill_f32_bytes(int M, int N, int K) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
-    const int64_t xb = align256((int64_t)M * K * 2);
-    const int64_t cb = align256((int64_t)N * (K / 128) * 8 * 4);
-    return 2 * xb + cb + prefill_split_bytes(M, N, K);
-}
-
-int launch_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed, const float* codebook,
-                       float* y, int64_t ldy, int M, int N, int K, void* workspace,
-                       int64_t ws_bytes, hipStream_t stream) {
-    unsigned char* w = static_cast<unsigned char*>(workspace);
-    const int64_t xb = align256((int64_t)M * K * 2);
-    const int64_t nent = (int64_t)N * (K / 128) * 8;
-    bf16_bits* hi = reinterpret_cast<bf16_bits*>(w);
-    bf16_bits* lo = reinterpret_cast<bf16_bits*>(w + xb);
-    float* cb_lo = reinterpret_cast<float*>(w + 2 * xb);
-    unsigned char* split = w + 2 * xb + align256(nent * 4);
-    const int64_t split_bytes = ws_bytes - (split - w);
-    const unsigned g1 = (unsigned)std::min<int64_t>(((int64_t)M * K + 255) / 256, 8192);
-    hipLaunchKernelGGL(split_bf16_kernel, dim3(g1), dim3(256), 0, stream, x, ldx, hi, lo, M, K);
-    const unsigned g2 = (unsigned)std::min<int64_t>((nent + 255) / 256, 4096);
-    hipLaunchKernelGGL(cb_residual_kernel, dim3(g2), dim3(256), 0, stream, codebook, cb_lo, nent);
-    int st = check_launch("nb_gemm_prefill_f32");
-    if (st) return st;
-    void* sw = split_bytes > 0 ? static_cast<void*>(split) : nullptr;
-    // x.W ~= hi.bf16(cb) + hi.bf16(cb_lo) + lo.bf16(cb), each pass in fp32,
-    // added to y in that order
-    st = launch_prefill2(hi, K, packed, codebook, y, NB_F32, ldy, M, N, K, sw, split_bytes, stream,
-                         false);
-    if (st) return st;
-    st = launch_prefill2(hi, K, packed, cb_lo, y, NB_F32, ldy, M, N, K, sw, split_bytes, stream,
-                         true);
-    if (st) return st;
-    return launch_prefill2(lo, K, packed, codebook, y, NB_F32, ldy, M, N, K, sw, split_bytes,
-                           stream, true);
-}
-
 int64_t prefill_split_bytes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
     const PrefillPlan p = prefill_plan(M, N, K, true);
     return p.S > 1 ? (int64_t)p.S * M * N * 4 : 0;
 }
 
-int launch_prefill2(const void* x, int64_t ldx, const uint8_t* packed, const float* codebook,
-                    void* y, int y_dtype, int64_t ldy, int M, int N, int K, void* workspace,
-                    int64_t ws_bytes, hipStream_t stream, bool accumulate) {
-    Prefill2Args a;
-    a.accumulate = accumulate ? 1 : 0;
-    a.x = static_cast<const uint16_t*>(x);
-    a.ldx = ldx;
-    a.packed = packed;
-    a.codebook = codebook;
-    a.y = y;
-    a.ldy = ldy;
-    a.y_dtype = y_dtype;
-    a.M = M;
-    a.N = N;
-    a.K = K;
-    PrefillPlan p = prefill_plan(M, N, K, workspace != nullptr);
-    if (p.S > 1 && ws_bytes < (int64_t)p.S * M * N * 4) p = prefill_plan(M, N, K, false);
+namespace {
+
+// The tiles of a plan, then the sum of their K ranges.
+template <bool kSplit>
+int launch_tiles(Prefill2Args a, const PrefillPlan& p, void* workspace, hipStream_t stream) {
     a.ksplit = p.S;
     a.part = p.S > 1 ? static_cast<float*>(workspace) : nullptr;
     constexpr int W = NB_PREFILL_WAVES;
+    const int M = a.M, N = a.N;
     const unsigned grid = (unsigned)(((N + p.BN - 1) / p.BN) * ((M + p.BM - 1) / p.BM) * p.S);
 #define NB_PREFILL2_LAUNCH(BMv, BNv)                                                          \
-    hipLaunchKernelGGL((prefill2_kernel<BMv, BNv, W>), dim3(grid), dim3(64 * W),             \
+    hipLaunchKernelGGL((prefill2_kernel<BMv, BNv, W, kSplit>), dim3(grid), dim3(64 * W),     \
                        (size_t)2 * (BMv + BNv) * kRowBytes, stream, a)
-    if (p.BM == 256 && p.BN == 256) {
-        NB_PREFILL2_LAUNCH(256, 256);
+    if (p.BN == 256) {
+        if constexpr (!kSplit) NB_PREFILL2_LAUNCH(256, 256);   // (not in kF32Tiles)
     } else if (p.BM == 256) {
         NB_PREFILL2_LAUNCH(256, 128);
     } else if (p.BM == 128) {
@@ -562,12 +619,73 @@ int launch_prefill2(const void* x, int64_t ldx, const uint8_t* packed, const flo
     if (p.S > 1) {
         const int st = check_launch("nb_gemm_prefill");
         if (st) return st;
-        const int64_t items = ((N | ldy) & 3) == 0 ? (int64_t)M * N / 4 : (int64_t)M * N;
+        const int64_t items = ((N | a.ldy) & 3) == 0 ? (int64_t)M * N / 4 : (int64_t)M * N;
         const unsigned rg = (unsigned)std::min<int64_t>((items + 255) / 256, 4096);
         hipLaunchKernelGGL(prefill_reduce_kernel, dim3(rg), dim3(256), 0, stream, a.part, p.S,
-                           M, N, y, y_dtype, ldy, a.accumulate);
+                           M, N, a.y, a.y_dtype, a.ldy);
     }
     return check_launch("nb_gemm_prefill");
+}
+
+}  // namespace
+
+int launch_prefill2(const void* x, int64_t ldx, const uint8_t* packed, const float* codebook,
+                    void* y, int y_dtype, int64_t ldy, int M, int N, int K, void* workspace,
+                    int64_t ws_bytes, hipStream_t stream) {
+    PrefillPlan p = prefill_plan(M, N, K, workspace != nullptr);
+    if (p.S > 1 && ws_bytes < (int64_t)p.S * M * N * 4) p = prefill_plan(M, N, K, false);
+    return launch_tiles<false>({static_cast<const uint16_t*>(x), ldx, packed, codebook, y, ldy,
+                                y_dtype, M, N, K, 1, nullptr}, p, workspace, stream);
+}
+
+int64_t prefill_f32_bytes(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
+    // (the size that callers may have stored: two bf16 parts of x, a codebook
+    // and the bf16 kernel's partial products; the codebook's part goes to
+    // partial products too)
+    const int64_t xb = align256((int64_t)M * K * 2);
+    const int64_t cb = align256((int64_t)N * (K / 128) * 8 * 4);
+    return 2 * xb + cb + prefill_split_bytes(M, N, K);
+}
+
+int launch_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed, const float* codebook,
+                       float* y, int64_t ldy, int M, int N, int K, void* workspace,
+                       hipStream_t stream) {
+    GemvArgs rows;
+    rows.x = x;
+    rows.x_dtype = NB_F32;
+    rows.ldx = ldx;
+    rows.packed = packed;
+    rows.packed_bytes = packed_nbytes((int64_t)N * K, 3);
+    rows.codebook = codebook;
+    rows.y = y;
+    rows.y_dtype = NB_F32;
+    rows.ldy = ldy;
+    rows.M = M;
+    rows.N = N;
+    rows.K = K;
+    rows.bits = 3;
+    rows.n_entries = 8;
+    rows.block_size = 128;
+    // Few rows of a small layer: the exact products on fp32 MFMAs, one launch
+    // (2560 x 2560 at M = 17 / 48: 12 / 21 us; 7680 x 2560 at M = 17 / 32: 22
+    // / 30 us against 26 / 26 below)
+    if ((int64_t)M * N * K <= 400000000 && gemm_rows_f32_eligible(rows)) {
+        return launch_gemm_rows_f32(rows, stream);
+    }
+    unsigned char* w = static_cast<unsigned char*>(workspace);
+    bf16_bits* xs = reinterpret_cast<bf16_bits*>(w);
+    const int64_t xbytes = align256((int64_t)M * K * 4);
+    const unsigned g = (unsigned)std::min<int64_t>(((int64_t)M * (K / 8) + 255) / 256, 8192);
+    const bool vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 && ldx % 4 == 0;
+    hipLaunchKernelGGL(vec ? split_bf16_kernel<true> : split_bf16_kernel<false>, dim3(g), dim3(256),
+                       0, stream, x, ldx, xs, M, K);
+    const int st = check_launch("nb_gemm_prefill_f32");
+    if (st) return st;
+    return launch_tiles<true>({xs, 2 * (int64_t)K, packed, codebook, y, ldy, NB_F32, M, N, K, 1,
+                               nullptr},
+                              prefill_f32_plan(M, N, K, prefill_f32_bytes(M, N, K) - xbytes),
+                              w + xbytes, stream);
 }
 
 }  // namespace nb

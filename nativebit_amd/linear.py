@@ -12,8 +12,9 @@ default.  Differences, all deliberate:
   bf16 and fp16 x too); more rows of bf16 activations run the packed MFMA
   prefill kernels (bf16-rounded codebook values, the reference's bf16 path
   of eval_ppl.py:149-174 -- its fp32 batched branch rejects bf16 x); more
-  rows of fp32 x run the same MFMA kernels in three bf16 passes over the hi
-  and lo parts of x and W (fp32-level products); other formats gather W on
+  rows of fp32 x run the same MFMA kernels with three bf16 products over the
+  hi and lo parts of x and W (fp32-level products; few rows of a small layer
+  the exact fp32 products); other formats gather W on
   the device with the format kernel and multiply it densely, as the
   reference's batched branch does; nothing falls back silently -- a failure raises
   NativeBitError (the reference swallows every exception,
@@ -90,8 +91,8 @@ class PackedLinear(torch.nn.Module):
                                  out_dtype=self.out_dtype)
         elif self._standard():
             # the reference's fp32 batched branch (triton_kernel.py:258-275) on
-            # the packed MFMA kernels: three bf16 passes over the hi / lo parts
-            # of x and of the exact fp32 weights, W never materialised
+            # the packed MFMA kernels: three bf16 products over the hi / lo
+            # parts of x and of the exact fp32 weights, W never materialised
             y = ops.gemm_prefill_f32(x_flat.contiguous(), self.packed_indices, self.codebook,
                                      N, K).to(self.out_dtype)
         else:

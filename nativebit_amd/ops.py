@@ -411,8 +411,9 @@ def gemm_prefill_f32(x: torch.Tensor, packed: torch.Tensor, codebook: torch.Tens
                      K: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """y = x @ W.T for fp32 x (M, K) against the exact fp32 codebook values of
     a 3-bit / 8-entry / block-128 packed W (N x K), y fp32 (M, N):
-    nb_gemm_prefill_f32, three bf16 MFMA passes over the hi / lo parts of x
-    and W (each product to within 2^-16 of its size), the packed weight
+    nb_gemm_prefill_f32, three bf16 products over the hi / lo parts of x and
+    W (each product to within 2^-16 of its size; few rows of a small layer:
+    the exact fp32 products), the packed weight
     dequantized into LDS tiles, never materialised; a workspace from torch's
     allocator."""
     for name, t in (("x", x), ("packed", packed), ("codebook", codebook)):
