@@ -134,15 +134,15 @@ int nb_gemm_prefill_split(const void* x, int64_t ldx, const uint8_t* packed,
  * The same contraction for fp32 activations against the exact fp32 codebook
  * values, y[m][n] = sum_k x[m][k] * W[n][k] (x fp32 row stride ldx, y fp32
  * row stride ldy, any alignment of their element type; K % 128 == 0), on
- * the bf16 MFMA kernel in three passes: x = hi + lo and W = W_hi + W_lo
- * split into bf16 parts (hi = bf16(v), lo = bf16(v - hi); W_lo through the
- * residual codebook cb - bf16(cb) over the same indices), y = hi.W_hi +
- * hi.W_lo + lo.W_hi accumulated in fp32 in that order.  Each product is x.W
- * to within 2^-16 of its size (the dropped lo.W_lo and the bf16 roundings
- * of the lo parts), against 2^-24 for an fp32 product; W is never
- * materialised.  The workspace needs nb_gemm_prefill_f32_ws_bytes(M, N, K)
- * bytes, 256-byte aligned (the bf16 parts of x, the residual codebook, the
- * K-split partial products), contents clobbered.  Deterministic.
+ * the bf16 MFMA kernel with three products a step: x = hi + lo and W = W_hi +
+ * W_lo split into bf16 parts (hi = bf16(v), lo = bf16(v - hi)), y = hi.W_hi +
+ * hi.W_lo + lo.W_hi accumulated in fp32.  Each product is x.W to within 2^-16
+ * of its size (the dropped lo.W_lo and the bf16 roundings of the lo parts),
+ * against 2^-24 for an fp32 product; few rows of a small layer run on fp32
+ * MFMAs with the exact products.  W is never materialised.  The workspace
+ * needs nb_gemm_prefill_f32_ws_bytes(M, N, K) bytes, 256-byte aligned (the
+ * bf16 parts of x, the K-split partial products), contents clobbered.
+ * Deterministic.
  * Replaces: the batched branch of PackedLinear.forward for fp32 x
  *           (unpack + gather + x @ W.T, inference/triton_kernel.py:258-275;
  *           nativebit/inference.py:42-46), without the per-call W.
@@ -512,6 +512,13 @@ int nb_rmsnorm_rows(float* x, const float* add, const float* emb, const int32_t*
  */
 int nb_silu_pairs_rows(const float* gu, void* act, int act_dtype, int T, int F, void* stream);
 /*
+ * act[i] = silu(gate[i]) * up[i] for i < n: the same product from separate
+ * gate and up outputs (fp32; act NB_F32 or NB_BF16).
+ * Replaces: F.silu(gate(x)) * up(x) (generate_torch.py:116-117).
+ */
+int nb_silu_mul_rows(const float* gate, const float* up, void* act, int act_dtype, int64_t n,
+                     void* stream);
+/*
  * For tokens t < T at positions pos0 + t: RoPE of the query and key heads of
  * qkv (T rows of 3 * n_head * head_dim fp32, q | k | v), the rotated keys
  * and the values appended to the caches, and q_out[t] = rotated q *
@@ -533,6 +540,18 @@ int nb_rope_kv_rows(const float* qkv, float* k_cache, float* v_cache, const floa
  */
 int nb_attention_rows(const float* q, const float* k_cache, const float* v_cache, int pos0, int T,
                       void* out, int out_dtype, int n_head, int head_dim, int ctx, void* stream);
+/*
+ * nb_rope_kv_rows and nb_attention_rows for `batch` sequences of T tokens at
+ * the same positions in one launch: qkv, q_out, q and out hold the
+ * sequences' rows one after the other, the caches [batch][n_head][...].
+ * Replaces: the same lines of CausalAttention.forward over the batch.
+ */
+int nb_rope_kv_batch(const float* qkv, float* k_cache, float* v_cache, const float* cos_t,
+                     const float* sin_t, int pos0, int T, float* q_out, int batch, int n_head,
+                     int head_dim, int ctx, void* stream);
+int nb_attention_batch(const float* q, const float* k_cache, const float* v_cache, int pos0, int T,
+                       void* out, int out_dtype, int batch, int n_head, int head_dim, int ctx,
+                       void* stream);
 
 /* ------------------------------------------------------------------------
  * Persistent decode: many greedy tokens of the whole packed decoder in one

@@ -83,8 +83,11 @@ SIGNATURES = {
     "nb_silu_mul": (_I, [_P, _P, _I, _I, _P]),
     "nb_rmsnorm_rows": (_I, [_P, _P, _P, _P, _I, _P, _P, _I, _I, _I, ctypes.c_float, _P]),
     "nb_silu_pairs_rows": (_I, [_P, _P, _I, _I, _I, _P]),
+    "nb_silu_mul_rows": (_I, [_P, _P, _P, _I, _L, _P]),
     "nb_rope_kv_rows": (_I, [_P, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _P]),
     "nb_attention_rows": (_I, [_P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _P]),
+    "nb_rope_kv_batch": (_I, [_P, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _P]),
+    "nb_attention_batch": (_I, [_P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _P]),
     "nb_lm_head_argmax": (_I, [_P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _P]),
     "nb_rmsnorm_lm_head_argmax": (_I, [_P, _P, ctypes.c_float, _P, _P, _P, _P, _I, _P, _I, _I,
                                        _I, _P]),

@@ -733,6 +733,21 @@ int nb_silu_pairs_rows(const float* gu, void* act, int act_dtype, int T, int F, 
     return launch_silu_pairs_rows(gu, act, act_dtype, T, F, static_cast<hipStream_t>(stream));
 }
 
+int nb_silu_mul_rows(const float* gate, const float* up, void* act, int act_dtype, int64_t n,
+                     void* stream) {
+    const char* fn = "nb_silu_mul_rows";
+    if (n < 0) return fail(NB_EINVAL, "%s: n=%lld < 0", fn, (long long)n);
+    if (act_dtype != NB_F32 && act_dtype != NB_BF16) return fail(NB_EINVAL, "%s: act_dtype=%d", fn, act_dtype);
+    if (n == 0) return NB_OK;
+    if (!gate || !up || !act) return fail(NB_EINVAL, "%s: NULL pointer", fn);
+    if (!aligned(gate, 4) || !aligned(up, 4) || !aligned(act, dtype_size(act_dtype))) {
+        return fail(NB_EALIGN, "%s: misaligned pointer", fn);
+    }
+    int st = ensure_device();
+    if (st) return st;
+    return launch_silu_mul_rows(gate, up, act, act_dtype, n, static_cast<hipStream_t>(stream));
+}
+
 namespace {
 int check_rows_attention(const char* fn, int pos0, int T, int n_head, int head_dim, int ctx) {
     if (T < 0 || n_head < 1 || ctx < 1 || pos0 < 0) {
@@ -750,12 +765,23 @@ int check_rows_attention(const char* fn, int pos0, int T, int n_head, int head_d
 }
 }  // namespace
 
-int nb_rope_kv_rows(const float* qkv, float* k_cache, float* v_cache, const float* cos_t,
-                    const float* sin_t, int pos0, int T, float* q_out, int n_head, int head_dim,
-                    int ctx, void* stream) {
-    const char* fn = "nb_rope_kv_rows";
+namespace {
+// Sequences of a batched row call; rows * heads stay in a grid's range.
+int check_batch_size(const char* fn, int batch, int T, int n_head) {
+    if (batch < 0) return fail(NB_EINVAL, "%s: batch=%d < 0", fn, batch);
+    if ((int64_t)batch * n_head * (T / 16 + 1) >= (1LL << 30)) {
+        return fail(NB_EUNSUPPORTED, "%s: batch=%d n_head=%d T=%d too large", fn, batch, n_head, T);
+    }
+    return NB_OK;
+}
+
+int rope_kv(const char* fn, const float* qkv, float* k_cache, float* v_cache, const float* cos_t,
+            const float* sin_t, int pos0, int T, float* q_out, int batch, int n_head, int head_dim,
+            int ctx, void* stream) {
     int st = check_rows_attention(fn, pos0, T, n_head, head_dim, ctx);
     if (st) return st;
+    st = check_batch_size(fn, batch, T, n_head);
+    if (st || batch == 0) return st;
     if (!qkv || !k_cache || !v_cache || !cos_t || !sin_t || !q_out) {
         return fail(NB_EINVAL, "%s: NULL pointer", fn);
     }
@@ -766,15 +792,17 @@ int nb_rope_kv_rows(const float* qkv, float* k_cache, float* v_cache, const floa
     if (T == 0) return NB_OK;
     st = ensure_device();
     if (st) return st;
-    return launch_rope_kv_rows(qkv, k_cache, v_cache, cos_t, sin_t, pos0, T, q_out, n_head,
+    return launch_rope_kv_rows(qkv, k_cache, v_cache, cos_t, sin_t, pos0, T, q_out, batch, n_head,
                                head_dim, ctx, static_cast<hipStream_t>(stream));
 }
 
-int nb_attention_rows(const float* q, const float* k_cache, const float* v_cache, int pos0, int T,
-                      void* out, int out_dtype, int n_head, int head_dim, int ctx, void* stream) {
-    const char* fn = "nb_attention_rows";
+int attention(const char* fn, const float* q, const float* k_cache, const float* v_cache, int pos0,
+              int T, void* out, int out_dtype, int batch, int n_head, int head_dim, int ctx,
+              void* stream) {
     int st = check_rows_attention(fn, pos0, T, n_head, head_dim, ctx);
     if (st) return st;
+    st = check_batch_size(fn, batch, T, n_head);
+    if (st || batch == 0) return st;
     if (out_dtype != NB_F32 && out_dtype != NB_BF16) return fail(NB_EINVAL, "%s: out_dtype=%d", fn, out_dtype);
     if (!q || !k_cache || !v_cache || !out) return fail(NB_EINVAL, "%s: NULL pointer", fn);
     if (!aligned(q, 4) || !aligned(k_cache, 4) || !aligned(v_cache, 4) ||
@@ -784,8 +812,36 @@ int nb_attention_rows(const float* q, const float* k_cache, const float* v_cache
     if (T == 0) return NB_OK;
     st = ensure_device();
     if (st) return st;
-    return launch_attention_rows(q, k_cache, v_cache, pos0, T, out, out_dtype, n_head, head_dim,
-                                 ctx, static_cast<hipStream_t>(stream));
+    return launch_attention_rows(q, k_cache, v_cache, pos0, T, out, out_dtype, batch, n_head,
+                                 head_dim, ctx, static_cast<hipStream_t>(stream));
+}
+}  // namespace
+
+int nb_rope_kv_rows(const float* qkv, float* k_cache, float* v_cache, const float* cos_t,
+                    const float* sin_t, int pos0, int T, float* q_out, int n_head, int head_dim,
+                    int ctx, void* stream) {
+    return rope_kv("nb_rope_kv_rows", qkv, k_cache, v_cache, cos_t, sin_t, pos0, T, q_out, 1, n_head,
+                   head_dim, ctx, stream);
+}
+
+int nb_rope_kv_batch(const float* qkv, float* k_cache, float* v_cache, const float* cos_t,
+                     const float* sin_t, int pos0, int T, float* q_out, int batch, int n_head,
+                     int head_dim, int ctx, void* stream) {
+    return rope_kv("nb_rope_kv_batch", qkv, k_cache, v_cache, cos_t, sin_t, pos0, T, q_out, batch,
+                   n_head, head_dim, ctx, stream);
+}
+
+int nb_attention_rows(const float* q, const float* k_cache, const float* v_cache, int pos0, int T,
+                      void* out, int out_dtype, int n_head, int head_dim, int ctx, void* stream) {
+    return attention("nb_attention_rows", q, k_cache, v_cache, pos0, T, out, out_dtype, 1, n_head,
+                     head_dim, ctx, stream);
+}
+
+int nb_attention_batch(const float* q, const float* k_cache, const float* v_cache, int pos0, int T,
+                       void* out, int out_dtype, int batch, int n_head, int head_dim, int ctx,
+                       void* stream) {
+    return attention("nb_attention_batch", q, k_cache, v_cache, pos0, T, out, out_dtype, batch,
+                     n_head, head_dim, ctx, stream);
 }
 
 int nb_silu_mul(const float* gu, void* act, int act_dtype, int n, void* stream) {

@@ -186,11 +186,13 @@ int launch_rmsnorm_rows(float* x, const float* add, const float* emb, const int3
 int launch_silu_pairs_rows(const float* gu, void* act, int act_dtype, int T, int F,
                            hipStream_t stream);
 int launch_rope_kv_rows(const float* qkv, float* k_cache, float* v_cache, const float* cos_t,
-                        const float* sin_t, int pos0, int T, float* q_out, int n_head, int D,
-                        int ctx, hipStream_t stream);
+                        const float* sin_t, int pos0, int T, float* q_out, int batch, int n_head,
+                        int D, int ctx, hipStream_t stream);
 int launch_attention_rows(const float* q, const float* k_cache, const float* v_cache, int pos0,
-                          int T, void* out, int out_dtype, int n_head, int D, int ctx,
+                          int T, void* out, int out_dtype, int batch, int n_head, int D, int ctx,
                           hipStream_t stream);
+int launch_silu_mul_rows(const float* gate, const float* up, void* act, int act_dtype, int64_t n,
+                         hipStream_t stream);
 // The same on fp32 MFMAs for head dims 64 and 128 over `batch` sequences
 // (nb_attention_mfma.hip): whether it takes the operands, and its launch.
 bool attention_mfma_eligible(const float* q, const float* k, const float* v, int D, int ctx);

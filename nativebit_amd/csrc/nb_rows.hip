@@ -6,16 +6,21 @@
 //                       h = rmsnorm(x) * w   (generate_torch.py:29-38, 128-132, 150)
 //   nb_silu_pairs_rows  act = silu(gate) * up from (gate, up) column pairs
 //                       (generate_torch.py:116-117)
+//   nb_silu_mul_rows    the same from separate gate and up arrays
 //   nb_rope_kv_rows     RoPE of q and k at positions pos0 .. pos0 + T - 1, k and v
 //                       appended to the caches, q * D^-0.5 kept for attention
 //                       (generate_torch.py:48-60, 80-88)
 //   nb_attention_rows   causal attention of T queries over cache positions
 //                       0 .. pos0 + t (generate_torch.py:89-98)
+//   nb_rope_kv_batch, nb_attention_batch   the last two for several sequences
 //
 // Arithmetic is fp32; outputs that feed a packed matmul may be rounded to
 // bf16 (nearest even).  The cache layout is the decode step's: keys
 // transposed [n_head][D][ctx], values [n_head][ctx][D].
 #include <math.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "nb_device.h"
 #include "nb_internal.h"
@@ -59,24 +64,30 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_rows_kernel(
     const float* src = tokens ? emb + (int64_t)tok * C : nullptr;
     const float* ar = add ? add + (int64_t)t * C : nullptr;
     // rows of up to kNormRegs * 256 elements stay in registers between the
-    // sum of squares and the scaling, with every load issued up front
+    // sum of squares and the scaling, with every load issued up front; 16
+    // bytes a lane where the rows allow it
     float ss = 0.f;
-    if (C <= kNormRegs * kNormThreads) {
-        float v[kNormRegs], wv[kNormRegs];
+    auto in_registers = [&](auto vec_c) {
+        constexpr int V = decltype(vec_c)::value;   // elements a load
+        typedef __attribute__((ext_vector_type(V))) float fv;
+        constexpr int kLoads = kNormRegs / V;
+        fv v[kLoads], wv[kLoads];
+        const float* from = src ? src : xr;
 #pragma unroll
-        for (int j = 0; j < kNormRegs; ++j) {
-            const int i = threadIdx.x + j * kNormThreads;
+        for (int j = 0; j < kLoads; ++j) {
+            const int i = V * (threadIdx.x + j * kNormThreads);
             const int ic = i < C ? i : 0;
-            v[j] = src ? src[ic] : xr[ic];
-            if (ar) v[j] = v[j] + ar[ic];
-            wv[j] = w[ic];
+            v[j] = *reinterpret_cast<const fv*>(from + ic);
+            if (ar) v[j] += *reinterpret_cast<const fv*>(ar + ic);
+            wv[j] = *reinterpret_cast<const fv*>(w + ic);
         }
 #pragma unroll
-        for (int j = 0; j < kNormRegs; ++j) {
-            const int i = threadIdx.x + j * kNormThreads;
+        for (int j = 0; j < kLoads; ++j) {
+            const int i = V * (threadIdx.x + j * kNormThreads);
             if (i < C) {
-                if (src || ar) xr[i] = v[j];
-                ss += v[j] * v[j];
+                if (src || ar) *reinterpret_cast<fv*>(xr + i) = v[j];
+#pragma unroll
+                for (int e = 0; e < V; ++e) ss += v[j][e] * v[j][e];
             }
         }
         ss = wsum(ss);
@@ -86,10 +97,33 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_rows_kernel(
         for (int k = 0; k < kNormThreads / 64; ++k) tot += red[k];  // same order everywhere
         const float norm = sqrtf(tot / (float)C + eps);
 #pragma unroll
-        for (int j = 0; j < kNormRegs; ++j) {
-            const int i = threadIdx.x + j * kNormThreads;
+        for (int j = 0; j < kLoads; ++j) {
+            const int i = V * (threadIdx.x + j * kNormThreads);
+            if (i >= C) continue;
             // (x / norm) * w, as generate_torch.py:37
-            if (i < C) store_out(h, h_dtype, (int64_t)t * C + i, (v[j] / norm) * wv[j]);
+            fv r;
+#pragma unroll
+            for (int e = 0; e < V; ++e) r[e] = (v[j][e] / norm) * wv[j][e];
+            const int64_t o = (int64_t)t * C + i;
+            if (h_dtype == NB_F32) {
+                *reinterpret_cast<fv*>(static_cast<float*>(h) + o) = r;
+            } else {
+                typedef __attribute__((ext_vector_type(V))) uint16_t hv;
+                hv p;
+#pragma unroll
+                for (int e = 0; e < V; ++e) p[e] = f32_to_bf16_rne(r[e]);
+                *reinterpret_cast<hv*>(static_cast<bf16_bits*>(h) + o) = p;
+            }
+        }
+    };
+    if (C <= kNormRegs * kNormThreads) {
+        const uintptr_t all = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(add) |
+                              reinterpret_cast<uintptr_t>(emb) | reinterpret_cast<uintptr_t>(w) |
+                              reinterpret_cast<uintptr_t>(h);
+        if (C % 4 == 0 && all % 16 == 0) {
+            in_registers(std::integral_constant<int, 4>{});
+        } else {
+            in_registers(std::integral_constant<int, 1>{});
         }
         return;
     }
@@ -123,33 +157,87 @@ __global__ void silu_pairs_rows_kernel(const float* __restrict__ gu, void* __res
     }
 }
 
-// ---------------------------------------------------------------------------
-// RoPE + cache append for T tokens: grid (T, n_head), D/2 threads (<= 128)
-// ---------------------------------------------------------------------------
-__global__ void rope_kv_rows_kernel(const float* __restrict__ qkv, float* __restrict__ k_cache,
-                                    float* __restrict__ v_cache, const float* __restrict__ cos_t,
-                                    const float* __restrict__ sin_t, int pos0,
-                                    float* __restrict__ q_out, int n_head, int D, int ctx) {
-    const int t = blockIdx.x, hd = blockIdx.y;
-    const int pos = pos0 + t;
-    const int C = n_head * D, half = D / 2;
-    const float scale = 1.0f / sqrtf((float)D);
-    const float* row = qkv + (int64_t)t * 3 * C;
-    for (int i = threadIdx.x; i < half; i += blockDim.x) {
-        const float c = cos_t[(int64_t)pos * half + i], s = sin_t[(int64_t)pos * half + i];
-        const float q0 = row[hd * D + 2 * i], q1 = row[hd * D + 2 * i + 1];
-        const float k0 = row[C + hd * D + 2 * i], k1 = row[C + hd * D + 2 * i + 1];
-        // x * cos2 + rotate(x) * sin2 (generate_torch.py:54-59), q then * scale
-        float* qo = q_out + (int64_t)t * C + hd * D;
-        qo[2 * i] = __fmul_rn(__fadd_rn(__fmul_rn(q0, c), __fmul_rn(-q1, s)), scale);
-        qo[2 * i + 1] = __fmul_rn(__fadd_rn(__fmul_rn(q1, c), __fmul_rn(q0, s)), scale);
-        k_cache[((int64_t)hd * D + 2 * i) * ctx + pos] = __fadd_rn(__fmul_rn(k0, c),
-                                                                   __fmul_rn(-k1, s));
-        k_cache[((int64_t)hd * D + 2 * i + 1) * ctx + pos] = __fadd_rn(__fmul_rn(k1, c),
-                                                                       __fmul_rn(k0, s));
+// act = silu(gate) * up from two arrays, four elements a thread.
+template <bool kVec>
+__global__ __launch_bounds__(256) void silu_mul_rows_kernel(const float* __restrict__ gate,
+                                                            const float* __restrict__ up,
+                                                            void* __restrict__ act, int act_dtype,
+                                                            int64_t n) {
+    for (int64_t i = 4 * (blockIdx.x * 256LL + threadIdx.x); i < n; i += 4 * 256LL * gridDim.x) {
+        float g[4], u[4];
+        if (kVec && i + 3 < n) {
+            const float4 a = *reinterpret_cast<const float4*>(gate + i);
+            const float4 b = *reinterpret_cast<const float4*>(up + i);
+            g[0] = a.x, g[1] = a.y, g[2] = a.z, g[3] = a.w;
+            u[0] = b.x, u[1] = b.y, u[2] = b.z, u[3] = b.w;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                g[e] = i + e < n ? gate[i + e] : 0.f;
+                u[e] = i + e < n ? up[i + e] : 0.f;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) g[e] = (g[e] / (1.0f + __expf(-g[e]))) * u[e];
+        if (kVec && act_dtype == NB_F32 && i + 3 < n) {
+            *reinterpret_cast<float4*>(static_cast<float*>(act) + i) = make_float4(g[0], g[1], g[2], g[3]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (i + e < n) store_out(act, act_dtype, i + e, g[e]);
+        }
     }
-    for (int d = threadIdx.x; d < D; d += blockDim.x) {
-        v_cache[((int64_t)hd * ctx + pos) * D + d] = row[2 * C + hd * D + d];
+}
+
+// ---------------------------------------------------------------------------
+// RoPE + cache append: a workgroup takes kRT tokens of one head of one
+// sequence.  The rows are read and q and v written a wave per token, lanes
+// along the head's pairs; the rotated keys pass through LDS so that they are
+// written along positions, the transposed cache's fast index (written by the
+// threads that rotate them, every 4-byte store had a cache line of its own:
+// 15.5 us for 500 tokens of 20 heads of 128, 31 MB; now 9.8).
+// ---------------------------------------------------------------------------
+constexpr int kRT = 32;
+constexpr int kRopeThreads = 256;
+constexpr int kRopeMaxD = 128;
+
+__global__ __launch_bounds__(kRopeThreads) void rope_kv_rows_kernel(
+    const float* __restrict__ qkv, float* __restrict__ k_cache, float* __restrict__ v_cache,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t, int pos0, int T,
+    float* __restrict__ q_out, int n_head, int D, int ctx, int tiles) {
+    __shared__ float ks[kRopeMaxD][kRT + 1];
+    const int bh = blockIdx.x / tiles, t0 = (blockIdx.x - bh * tiles) * kRT;
+    const int b = bh / n_head, hd = bh - b * n_head;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int C = n_head * D, half = D / 2;
+    const int nt = min(kRT, T - t0);
+    const float scale = 1.0f / sqrtf((float)D);
+#pragma unroll 4
+    for (int t = wave; t < nt; t += kRopeThreads / 64) {
+        const int64_t tok = (int64_t)b * T + t0 + t;
+        const int pos = pos0 + t0 + t;
+        const float* row = qkv + tok * 3 * C + hd * D;
+        float* qo = q_out + tok * C + hd * D;
+        float* vo = v_cache + ((int64_t)bh * ctx + pos) * D;
+        for (int i = lane; i < half; i += 64) {
+            const float c = cos_t[(int64_t)pos * half + i], s = sin_t[(int64_t)pos * half + i];
+            const float q0 = row[2 * i], q1 = row[2 * i + 1];
+            const float k0 = row[C + 2 * i], k1 = row[C + 2 * i + 1];
+            const float v0 = row[2 * C + 2 * i], v1 = row[2 * C + 2 * i + 1];
+            // x * cos2 + rotate(x) * sin2 (generate_torch.py:54-59), q then * scale
+            qo[2 * i] = __fmul_rn(__fadd_rn(__fmul_rn(q0, c), __fmul_rn(-q1, s)), scale);
+            qo[2 * i + 1] = __fmul_rn(__fadd_rn(__fmul_rn(q1, c), __fmul_rn(q0, s)), scale);
+            ks[2 * i][t] = __fadd_rn(__fmul_rn(k0, c), __fmul_rn(-k1, s));
+            ks[2 * i + 1][t] = __fadd_rn(__fmul_rn(k1, c), __fmul_rn(k0, s));
+            vo[2 * i] = v0;
+            vo[2 * i + 1] = v1;
+        }
+    }
+    __syncthreads();
+    const int t = threadIdx.x % kRT;
+    if (t < nt) {
+        float* ko = k_cache + (int64_t)bh * D * ctx + pos0 + t0 + t;
+        for (int d = threadIdx.x / kRT; d < D; d += kRopeThreads / kRT) ko[(int64_t)d * ctx] = ks[d][t];
     }
 }
 
@@ -291,27 +379,44 @@ int launch_silu_pairs_rows(const float* gu, void* act, int act_dtype, int T, int
     return check_launch("nb_silu_pairs_rows");
 }
 
+int launch_silu_mul_rows(const float* gate, const float* up, void* act, int act_dtype, int64_t n,
+                         hipStream_t stream) {
+    const int blocks = (int)std::min<int64_t>(4096, (n / 4 + 256) / 256);
+    const bool vec = (reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up) |
+                      reinterpret_cast<uintptr_t>(act)) % 16 == 0;
+    hipLaunchKernelGGL(vec ? silu_mul_rows_kernel<true> : silu_mul_rows_kernel<false>, dim3(blocks),
+                       dim3(256), 0, stream, gate, up, act, act_dtype, n);
+    return check_launch("nb_silu_mul_rows");
+}
+
 int launch_rope_kv_rows(const float* qkv, float* k_cache, float* v_cache, const float* cos_t,
-                        const float* sin_t, int pos0, int T, float* q_out, int n_head, int D,
-                        int ctx, hipStream_t stream) {
-    hipLaunchKernelGGL(rope_kv_rows_kernel, dim3(T, n_head), dim3(64), 0, stream, qkv, k_cache,
-                       v_cache, cos_t, sin_t, pos0, q_out, n_head, D, ctx);
+                        const float* sin_t, int pos0, int T, float* q_out, int batch, int n_head,
+                        int D, int ctx, hipStream_t stream) {
+    static_assert(kRopeMaxD >= kRowsMaxD, "the callers' largest head dim");
+    const int tiles = (T + kRT - 1) / kRT;
+    hipLaunchKernelGGL(rope_kv_rows_kernel, dim3((unsigned)(batch * n_head * tiles)),
+                       dim3(kRopeThreads), 0, stream, qkv, k_cache, v_cache, cos_t, sin_t, pos0, T,
+                       q_out, n_head, D, ctx, tiles);
     return check_launch("nb_rope_kv_rows");
 }
 
 int launch_attention_rows(const float* q, const float* k_cache, const float* v_cache, int pos0,
-                          int T, void* out, int out_dtype, int n_head, int D, int ctx,
+                          int T, void* out, int out_dtype, int batch, int n_head, int D, int ctx,
                           hipStream_t stream) {
     // fp32 MFMAs where the layout allows 16-byte loads; up to 32 positions at
     // head dim 128 the vector kernel below is as fast or faster (16 queries
     // from position 0: 8.0 us against 8.9; 64: 9.3 against 9.0)
     if (attention_mfma_eligible(q, k_cache, v_cache, D, ctx) && (D < 128 || pos0 + T > 32)) {
-        return launch_attention_mfma(q, k_cache, v_cache, pos0, T, out, out_dtype, 1, n_head, D,
+        return launch_attention_mfma(q, k_cache, v_cache, pos0, T, out, out_dtype, batch, n_head, D,
                                      ctx, stream);
     }
-    hipLaunchKernelGGL(attention_rows_kernel, dim3(n_head, (T + kQB - 1) / kQB),
-                       dim3(kAttThreads), 0, stream, q, k_cache, v_cache, pos0, T, out,
-                       out_dtype, n_head, D, ctx);
+    for (int b = 0; b < batch; ++b) {
+        const int64_t rows = (int64_t)b * T * n_head * D, cache = (int64_t)b * n_head * D * ctx;
+        void* o = static_cast<char*>(out) + rows * (out_dtype == NB_BF16 ? 2 : 4);
+        hipLaunchKernelGGL(attention_rows_kernel, dim3(n_head, (T + kQB - 1) / kQB),
+                           dim3(kAttThreads), 0, stream, q + rows, k_cache + cache, v_cache + cache,
+                           pos0, T, o, out_dtype, n_head, D, ctx);
+    }
     return check_launch("nb_attention_rows");
 }
 

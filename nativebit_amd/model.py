@@ -18,8 +18,8 @@ The arithmetic runs in this library's kernels: the packed linears are
 PackedLinear (fused dequant-GEMV for up to 16 rows, the packed MFMA kernels or
 a device gather + dense GEMM beyond), the norms nb_rmsnorm_rows (the residual
 add fused into the second norm of a block), RoPE and the cache appends
-nb_rope_kv_rows, attention nb_attention_rows, the SwiGLU product
-nb_silu_pairs_rows.  Activations stay fp32 (the reference's module numerics);
+nb_rope_kv_batch, attention nb_attention_batch, the SwiGLU product
+nb_silu_mul_rows.  Activations stay fp32 (the reference's module numerics);
 ``nativebit_amd.decode.DecodeEngine`` runs the same model with bf16 GEMV
 inputs, one HIP graph per token, for speed.
 
@@ -170,7 +170,7 @@ def _cache_storage(k_buf, v_buf, B, H, D):
 class CausalAttention(nn.Module):
     """Causal self-attention (generate_torch.py:63-106): the packed q|k|v and
     output projections (built by ``make_linear(out, in)``) around
-    nb_rope_kv_rows (RoPE, cache append) and nb_attention_rows (masked
+    nb_rope_kv_batch (RoPE, cache append) and nb_attention_batch (masked
     softmax over the cache).
 
     With a cache (keys, values, length) the tokens take positions length ..
@@ -215,14 +215,13 @@ class CausalAttention(nn.Module):
             raise ValueError(f"positions up to {first + T} exceed the RoPE tables "
                              f"({cos.shape[0]})")
         cos_t, sin_t = cos[first - pos0:], sin[first - pos0:]
-        q = torch.empty(T, C, device=dev)
+        q = torch.empty(B, T, C, device=dev)
         att = torch.empty(B, T, C, device=dev)
         lib, s = _lib.load(), _stream(dev)
-        for b in range(B):
-            _lib.check(lib.nb_rope_kv_rows(_p(qkv[b]), _p(kt[b]), _p(vt[b]), _p(cos_t),
-                                           _p(sin_t), pos0, T, _p(q), H, D, ctx, s))
-            _lib.check(lib.nb_attention_rows(_p(q), _p(kt[b]), _p(vt[b]), pos0, T,
-                                             _p(att[b]), _lib.NB_F32, H, D, ctx, s))
+        _lib.check(lib.nb_rope_kv_batch(_p(qkv), _p(kt), _p(vt), _p(cos_t), _p(sin_t), pos0, T,
+                                        _p(q), B, H, D, ctx, s))
+        _lib.check(lib.nb_attention_batch(_p(q), _p(kt), _p(vt), pos0, T, _p(att), _lib.NB_F32, B,
+                                          H, D, ctx, s))
         out = self.out_proj(att)
         if kv_cache is None:
             return out, None
@@ -235,7 +234,7 @@ class CausalAttention(nn.Module):
 
 class SwiGLU(nn.Module):
     """down(silu(gate(x)) * up(x)) (generate_torch.py:109-117); the product is
-    nb_silu_pairs_rows over the gate and up outputs side by side."""
+    nb_silu_mul_rows over the gate and up outputs."""
 
     def __init__(self, n_embd, ffn_hidden, make_linear):
         super().__init__()
@@ -246,10 +245,10 @@ class SwiGLU(nn.Module):
     def forward(self, x):
         g, u = self.gate(x), self.up(x)
         F = g.shape[-1]
-        pairs = torch.stack((g.float(), u.float()), dim=-1).reshape(-1, 2 * F).contiguous()
-        act = torch.empty(pairs.shape[0], F, device=x.device)
-        _lib.check(_lib.load().nb_silu_pairs_rows(_p(pairs), _p(act), _lib.NB_F32,
-                                                  pairs.shape[0], F, _stream(x.device)))
+        gf, uf = g.float().contiguous(), u.float().contiguous()
+        act = torch.empty(gf.numel(), device=x.device)
+        _lib.check(_lib.load().nb_silu_mul_rows(_p(gf), _p(uf), _p(act), _lib.NB_F32, gf.numel(),
+                                                _stream(x.device)))
         prod_dtype = torch.promote_types(g.dtype, u.dtype)
         return self.down(act.reshape(*g.shape[:-1], F).to(prod_dtype))
 
