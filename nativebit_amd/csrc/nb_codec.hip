@@ -271,76 +271,159 @@ __global__ __launch_bounds__(64) void block_codebooks_kernel(
     }
 }
 
-// The same codebooks for blocks of at most 64 * H weights, sorted in one
-// wave's registers: value i of the (+inf padded) block sits in lane i % 64,
-// slot i / 64; each bitonic pass pairs i with i ^ j (a cross-lane shuffle for
-// j < 64, another slot of the same lane otherwise) and keeps the min or the
-// max, so no LDS and no barrier is involved.  Entries are then formed as in
-// block_codebooks_kernel from values fetched by shuffles.
-template <int H>
-__device__ __forceinline__ float sorted_at(const float (&v)[H], int idx) {
-    float r = __shfl(v[0], idx & 63, 64);
-#pragma unroll
-    for (int h = 1; h < H; ++h) {
-        const float u = __shfl(v[h], idx & 63, 64);
-        r = (idx >> 6) == h ? u : r;
-    }
+// The same codebooks for blocks of at most 16 * R weights, four blocks a
+// wave: sorted value i of a block is slot i % R of lane i / R of a 16-lane
+// row, so every pass of the sorting network stays within a lane or a DPP row
+// (no LDS, no barrier, no ds_bpermute).  Each lane sorts its R values (odd-
+// even merge sort); then lane groups of 2, 4, 8 and 16 are merged: a group's
+// first pass pairs lane l with its mirror image and slot r with R - 1 - r, the
+// next ones lanes 4, 2, 1 apart, the last ones slots of a lane, the smaller
+// value always to the smaller index.  A pass across lanes is a DPP move and a
+// three-way median with the smallest or largest key (the smaller or larger
+// of the two); values are compared as integers of the same order (-0 below
+// +0).  What bounds it: 302 sorting instructions per four 128-weight blocks,
+// 17 us over 138 240 blocks at full issue, beside 12 us of reads.  Measured
+// (6912 x 2560): see launch_block_codebooks.
+__device__ __forceinline__ int sort_key(float f) {
+    const int i = __float_as_int(f);
+    return i ^ ((i >> 31) & 0x7fffffff);
+}
+__device__ __forceinline__ float sort_value(int k) {
+    return __int_as_float(k ^ ((k >> 31) & 0x7fffffff));
+}
+
+__device__ __forceinline__ int med3(int a, int b, int c) {
+    int r;
+    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
 
-template <int H>
-__global__ __launch_bounds__(kThreads) void block_codebooks_wave_kernel(
+// The value of lane l ^ X of the row (X = 1, 2, 3, 4, 7 or 15).
+template <int X>
+__device__ __forceinline__ int row_xor(int v) {
+    if constexpr (X == 4) {   // lanes 0-3 and 8-11 take lane + 4, the others lane - 4
+        const int up = __builtin_amdgcn_update_dpp(v, v, 0x104, 0xf, 0x5, false);
+        return __builtin_amdgcn_update_dpp(up, v, 0x114, 0xf, 0xa, false);
+    } else {
+        constexpr int ctrl = X == 1 ? 0xB1 : X == 2 ? 0x4E : X == 3 ? 0x1B : X == 7 ? 0x141 : 0x140;
+        return __builtin_amdgcn_mov_dpp(v, ctrl, 0xf, 0xf, false);
+    }
+}
+
+__device__ __forceinline__ void order2(int& a, int& b) {
+    const int lo = min(a, b), hi = max(a, b);
+    a = lo;
+    b = hi;
+}
+
+// Merges sorted runs of G / 2 lanes into runs of G lanes.
+template <int R, int G>
+__device__ __forceinline__ void merge_lanes(int (&v)[R], int lane) {
+    int o[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) o[r] = row_xor<G - 1>(v[R - 1 - r]);
+    int c = lane & (G / 2) ? INT32_MAX : INT32_MIN;
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = med3(v[r], o[r], c);
+    auto apart = [&](auto dc) {
+        constexpr int d = decltype(dc)::value;
+        c = lane & d ? INT32_MAX : INT32_MIN;
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = med3(v[r], row_xor<d>(v[r]), c);
+    };
+    if constexpr (G >= 16) apart(std::integral_constant<int, 4>{});
+    if constexpr (G >= 8) apart(std::integral_constant<int, 2>{});
+    if constexpr (G >= 4) apart(std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int d = R / 2; d > 0; d >>= 1) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (!(r & d)) order2(v[r], v[r + d]);
+    }
+}
+
+template <int R>
+__global__ __launch_bounds__(kThreads) void block_codebooks_row_kernel(
     const float* __restrict__ w, int64_t total, int64_t num_blocks, int block_size, int n_entries,
-    QuantileFractions qf, float* __restrict__ cb) {
-    constexpr int P = 64 * H;
-    const int lane = threadIdx.x & 63;
-    const int64_t nwaves = ((int64_t)gridDim.x * kThreads) >> 6;
-    for (int64_t b = ((int64_t)blockIdx.x * kThreads + threadIdx.x) >> 6; b < num_blocks;
-         b += nwaves) {
+    bool vec, QuantileFractions qf, float* __restrict__ cb) {
+    constexpr int P = 16 * R;
+    __shared__ __align__(16) int sorted[kThreads / 16][P];
+    const int lane = threadIdx.x & 15, row = threadIdx.x >> 4;
+    const int64_t nrows = ((int64_t)gridDim.x * kThreads) >> 4;
+    // (rows past the last block repeat it and store nothing: every lane of a
+    // wave takes part in the DPP moves)
+    const int64_t rounds = (num_blocks + nrows - 1) / nrows;
+    for (int64_t it = 0; it < rounds; ++it) {
+        const int64_t b0 = it * nrows + (((int64_t)blockIdx.x * kThreads + threadIdx.x) >> 4);
+        const int64_t b = b0 < num_blocks ? b0 : num_blocks - 1;
         const int64_t first = b * block_size;
         const int n = (int)min((int64_t)block_size, total - first);
-        float v[H];
+        int v[R];
+        if (vec && n == P) {
 #pragma unroll
-        for (int h = 0; h < H; ++h) {
-            const int i = lane + 64 * h;
-            v[h] = i < n ? w[first + i] : INFINITY;
+            for (int q = 0; q < R / 4; ++q) {
+                const float4 f = reinterpret_cast<const float4*>(w + first)[q * 16 + lane];
+                v[4 * q] = sort_key(f.x);
+                v[4 * q + 1] = sort_key(f.y);
+                v[4 * q + 2] = sort_key(f.z);
+                v[4 * q + 3] = sort_key(f.w);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int i = r * 16 + lane;
+                v[r] = sort_key(i < n ? w[first + i] : INFINITY);
+            }
         }
+        // the lane's own values: odd-even merge sort
 #pragma unroll
-        for (int k = 2; k <= P; k <<= 1) {
+        for (int p = 1; p < R; p <<= 1) {
 #pragma unroll
-            for (int j = k >> 1; j > 0; j >>= 1) {
-                float o[H];
+            for (int k = p; k >= 1; k >>= 1) {
 #pragma unroll
-                for (int h = 0; h < H; ++h) {
-                    o[h] = j < 64 ? __shfl_xor(v[h], j, 64) : v[h ^ (j >> 6)];
-                }
+                for (int j = k % p; j + k < R; j += 2 * k) {
 #pragma unroll
-                for (int h = 0; h < H; ++h) {
-                    const int i = lane + 64 * h;
-                    const bool keep_min = ((i & j) == 0) == ((i & k) == 0);
-                    v[h] = keep_min ? fminf(v[h], o[h]) : fmaxf(v[h], o[h]);
+                    for (int i = 0; i < k; ++i) {
+                        if (i + j + k < R && (i + j) / (2 * p) == (i + j + k) / (2 * p)) {
+                            order2(v[i + j], v[i + j + k]);
+                        }
+                    }
                 }
             }
         }
+        merge_lanes<R, 2>(v, lane);
+        merge_lanes<R, 4>(v, lane);
+        merge_lanes<R, 8>(v, lane);
+        merge_lanes<R, 16>(v, lane);
+        // entries: a lane fetches its two order statistics through LDS (a
+        // wave's LDS operations complete in issue order)
+#pragma unroll
+        for (int q = 0; q < R / 4; ++q) {
+            *reinterpret_cast<int4*>(&sorted[row][lane * R + 4 * q]) =
+                make_int4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const float last_index = (float)(n - 1);
-        for (int e0 = 0; e0 < n_entries; e0 += 64) {  // uniform: every lane shuffles
-            const int e = e0 + lane;
+        for (int e = lane; e < n_entries; e += 16) {
             float rank, wt;
             int lo, hi;
             {
                 // each product and difference rounded on its own, as torch's
                 // CPU quantile computes them: no contraction into fma here
 #pragma clang fp contract(off)
-                rank = qf.q[e < n_entries ? e : 0] * last_index;
+                rank = qf.q[e] * last_index;
                 lo = (int)rank;
                 hi = (int)ceilf(rank);
                 wt = rank - (float)lo;
             }
-            const float a = sorted_at<H>(v, lo), c = sorted_at<H>(v, hi);
+            const float a = sort_value(sorted[row][lo]), c = sort_value(sorted[row][hi]);
             const float r = fabsf(wt) < 0.5f ? __builtin_fmaf(wt, c - a, a)
                                              : __builtin_fmaf(wt - 1.0f, c - a, c);
-            if (e < n_entries) cb[b * n_entries + e] = r;
+            if (b0 < num_blocks) cb[b * n_entries + e] = r;
         }
+        __builtin_amdgcn_wave_barrier();   // (the next blocks' writes stay behind these reads)
     }
 }
 
@@ -638,19 +721,22 @@ int launch_block_codebooks(const float* w, int64_t total, int64_t num_blocks, in
     QuantileFractions qf;
     for (int e = 0; e < kCbMaxEntries; ++e) qf.q[e] = e < n_entries ? q[e] : 0.f;
     if (block_size <= 256) {
-        const int64_t want = (num_blocks + kThreads / 64 - 1) / (kThreads / 64);
-        const int64_t cap = (int64_t)device_cu_count() * 16;
+        // 6912 x 2560, 8 entries: 98 us with one block a wave sorted by
+        // ds_bpermute shuffles, 31 us with four (70.8 MB read: 2.4 TB/s)
+        const int64_t want = (num_blocks + kThreads / 16 - 1) / (kThreads / 16);
+        const int64_t cap = (int64_t)device_cu_count() * 8;
         const int grid = (int)(want < cap ? want : cap);
+        const bool vec = is_aligned(w, 16) && block_size % 4 == 0;
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, stream, w, total,
-                               num_blocks, block_size, n_entries, qf, cb);
+                               num_blocks, block_size, n_entries, vec, qf, cb);
         };
         if (block_size <= 64) {
-            go(block_codebooks_wave_kernel<1>);
+            go(block_codebooks_row_kernel<4>);
         } else if (block_size <= 128) {
-            go(block_codebooks_wave_kernel<2>);
+            go(block_codebooks_row_kernel<8>);
         } else {
-            go(block_codebooks_wave_kernel<4>);
+            go(block_codebooks_row_kernel<16>);
         }
         return check_launch("nb_block_codebooks");
     }
