@@ -71,9 +71,11 @@ class PackedLinear(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         shape = x.shape
-        if x.dim() == 0 or shape[-1] != self.in_features:
-            raise ValueError(f"x last dim must be {self.in_features}, got {tuple(shape)}")
-        x_flat = x.reshape(-1, self.in_features)
+        N, K = self.out_features, self.in_features
+        if x.dim() == 0 or shape[-1] != K:
+            raise ValueError(f"x last dim must be {K}, got {tuple(shape)}")
+        flat = len(shape) == 2
+        x_flat = x if flat else x.reshape(-1, K)
         M = x_flat.shape[0]
         if x_flat.dtype != torch.float32 and (M <= MAX_GEMV_ROWS or
                                               x_flat.dtype != torch.bfloat16):
@@ -81,10 +83,10 @@ class PackedLinear(torch.nn.Module):
             # fp32 codebook values, as the reference's batch-1 kernels compute
             # (.to(tl.float32), triton_kernel.py:46, 174-183)
             x_flat = x_flat.to(torch.float32)
-        N, K = self.out_features, self.in_features
         if M <= MAX_GEMV_ROWS:
-            y = ops.gemv(x_flat, self.packed_indices, self.codebook, N, K, bits=self.bits,
-                         block_size=self.block_size, out_dtype=self.out_dtype)
+            buffers = self._buffers   # (nn.Module's attribute lookup, 0.3 us each)
+            y = ops.gemv(x_flat, buffers["packed_indices"], buffers["codebook"], N, K,
+                         bits=self.bits, block_size=self.block_size, out_dtype=self.out_dtype)
         elif x_flat.dtype == torch.bfloat16 and self._standard():
             # the bf16 batched form (eval_ppl.py:149-174): the packed MFMA kernels
             y = ops.gemm_prefill(x_flat, self.packed_indices, self.codebook, N, K,
@@ -103,7 +105,7 @@ class PackedLinear(torch.nn.Module):
             w = ops.dequant(self.packed_indices, self.codebook, N * K, self.bits,
                             self.block_size, x_flat.dtype).view(N, K)
             y = (x_flat @ w.T).to(self.out_dtype)
-        return y.reshape(*shape[:-1], N)
+        return y if flat else y.reshape(*shape[:-1], N)
 
     @staticmethod
     def from_packed(indices_np, codebook_np, weight_shape, device="cuda",

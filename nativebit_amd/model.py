@@ -33,7 +33,6 @@ kernel layout for the call and the new positions written back.
 """
 from __future__ import annotations
 
-import ctypes
 import itertools
 from dataclasses import dataclass
 
@@ -43,6 +42,7 @@ import torch.nn as nn
 
 from . import _lib, formats, synth
 from .linear import PackedLinear
+from .ops import _stream
 
 
 @dataclass
@@ -86,17 +86,15 @@ def model_config(config) -> ModelConfig:
                        norm_eps=float(getattr(config, "norm_eps", 1e-6)))
 
 
-def _stream(dev) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-
-
 def _p(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
-def _rows(x: torch.Tensor, width: int) -> torch.Tensor:
-    """x as contiguous fp32 rows of `width` (a copy when it is not already)."""
-    return x.reshape(-1, width).to(torch.float32).contiguous()
+def _f32(t: torch.Tensor) -> torch.Tensor:
+    """t in contiguous fp32 (a copy when it is not already)."""
+    if t.dtype == torch.float32 and t.is_contiguous():
+        return t
+    return t.to(torch.float32).contiguous()
 
 
 class RMSNorm(nn.Module):
@@ -111,13 +109,13 @@ class RMSNorm(nn.Module):
 
     def forward(self, x):
         C = x.shape[-1]
-        rows = _rows(x, C)
+        rows = _f32(x)
         out = torch.empty_like(rows)
-        w = self.weight.detach().to(torch.float32).contiguous()
+        w = _f32(self.weight.detach())
         _lib.check(_lib.load().nb_rmsnorm_rows(
-            _p(rows), None, None, None, 0, _p(w), _p(out), _lib.NB_F32, rows.shape[0], C,
-            float(self.eps), _stream(x.device)))
-        return out.reshape(x.shape).to(x.dtype)
+            _p(rows), None, None, None, 0, _p(w), _p(out), _lib.NB_F32, rows.numel() // C, C,
+            float(self.eps), _stream(rows)))
+        return out.to(x.dtype)
 
 
 def precompute_rope(dim, max_len, theta=10000.0):
@@ -196,8 +194,10 @@ class CausalAttention(nn.Module):
         B, T, C = x.shape
         H, D = self.n_head, self.head_dim
         dev = x.device
-        qkv = self.qkv(x).reshape(B, T, 3 * C).to(torch.float32).contiguous()
-        cos, sin = self.cos.to(dev).contiguous(), self.sin.to(dev).contiguous()
+        qkv = _f32(self.qkv(x))
+        if qkv.shape != (B, T, 3 * C):
+            qkv = qkv.reshape(B, T, 3 * C)
+        cos, sin = _f32(self.cos.to(dev)), _f32(self.sin.to(dev))
         if kv_cache is not None:
             k_buf, v_buf, pos0 = kv_cache
             pos0 = int(pos0)
@@ -206,19 +206,22 @@ class CausalAttention(nn.Module):
             if pos0 < 0 or pos0 + T > ctx:
                 raise ValueError(f"positions {pos0}..{pos0 + T - 1} outside a cache of {ctx}")
         else:
-            # the T tokens alone: a scratch cache of T positions, RoPE tables
-            # read from row pos_offset on
-            kt = torch.zeros(B, H, D, T, device=dev)
-            vt = torch.zeros(B, H, T, D, device=dev)
-            pos0, ctx, first = 0, T, int(pos_offset)
+            # the T tokens alone: a scratch cache of T positions (rows of keys
+            # padded to 16 bytes; nothing past T is used), RoPE tables read
+            # from row pos_offset on
+            ctx = (T + 3) // 4 * 4
+            kt = torch.empty(B, H, D, ctx, device=dev)
+            vt = torch.empty(B, H, ctx, D, device=dev)
+            pos0, first = 0, int(pos_offset)
         if first < 0 or first + T > cos.shape[0]:
             raise ValueError(f"positions up to {first + T} exceed the RoPE tables "
                              f"({cos.shape[0]})")
-        cos_t, sin_t = cos[first - pos0:], sin[first - pos0:]
+        if first != pos0:
+            cos, sin = cos[first - pos0:], sin[first - pos0:]
         q = torch.empty(B, T, C, device=dev)
         att = torch.empty(B, T, C, device=dev)
-        lib, s = _lib.load(), _stream(dev)
-        _lib.check(lib.nb_rope_kv_batch(_p(qkv), _p(kt), _p(vt), _p(cos_t), _p(sin_t), pos0, T,
+        lib, s = _lib.load(), _stream(qkv)
+        _lib.check(lib.nb_rope_kv_batch(_p(qkv), _p(kt), _p(vt), _p(cos), _p(sin), pos0, T,
                                         _p(q), B, H, D, ctx, s))
         _lib.check(lib.nb_attention_batch(_p(q), _p(kt), _p(vt), pos0, T, _p(att), _lib.NB_F32, B,
                                           H, D, ctx, s))
@@ -244,13 +247,11 @@ class SwiGLU(nn.Module):
 
     def forward(self, x):
         g, u = self.gate(x), self.up(x)
-        F = g.shape[-1]
-        gf, uf = g.float().contiguous(), u.float().contiguous()
-        act = torch.empty(gf.numel(), device=x.device)
+        gf, uf = _f32(g), _f32(u)
+        act = torch.empty_like(gf)
         _lib.check(_lib.load().nb_silu_mul_rows(_p(gf), _p(uf), _p(act), _lib.NB_F32, gf.numel(),
-                                                _stream(x.device)))
-        prod_dtype = torch.promote_types(g.dtype, u.dtype)
-        return self.down(act.reshape(*g.shape[:-1], F).to(prod_dtype))
+                                                _stream(gf)))
+        return self.down(act.to(torch.promote_types(g.dtype, u.dtype)))
 
 
 class TransformerBlock(nn.Module):
@@ -273,10 +274,10 @@ class TransformerBlock(nn.Module):
         x1_dtype = torch.promote_types(x.dtype, a.dtype)
         res = x.reshape(-1, C).to(torch.float32, copy=True)   # becomes x + a (a fresh copy)
         h = torch.empty_like(res)
-        w2 = self.ln2.weight.detach().to(torch.float32).contiguous()
+        w2, add = _f32(self.ln2.weight.detach()), _f32(a)
         _lib.check(_lib.load().nb_rmsnorm_rows(
-            _p(res), _p(_rows(a, C)), None, None, 0, _p(w2), _p(h), _lib.NB_F32, res.shape[0], C,
-            float(self.ln2.eps), _stream(x.device)))
+            _p(res), _p(add), None, None, 0, _p(w2), _p(h), _lib.NB_F32, res.shape[0], C,
+            float(self.ln2.eps), _stream(res)))
         res = res.reshape(x.shape).to(x1_dtype)
         f = self.ffn(h.reshape(x.shape).to(x1_dtype))
         return res + f, new_cache
