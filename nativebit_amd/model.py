@@ -247,6 +247,8 @@ class SwiGLU(nn.Module):
 
     def forward(self, x):
         g, u = self.gate(x), self.up(x)
+        if g.shape != u.shape or g.device != u.device:   # (the kernel walks both by one count)
+            raise RuntimeError(f"gate {tuple(g.shape)} on {g.device}, up {tuple(u.shape)} on {u.device}")
         gf, uf = _f32(g), _f32(u)
         act = torch.empty_like(gf)
         _lib.check(_lib.load().nb_silu_mul_rows(_p(gf), _p(uf), _p(act), _lib.NB_F32, gf.numel(),
@@ -271,6 +273,8 @@ class TransformerBlock(nn.Module):
     def forward(self, x, kv_cache=None, pos_offset=0):
         C = x.shape[-1]
         a, new_cache = self.attn(self.ln1(x), kv_cache, pos_offset=pos_offset)
+        if a.numel() != x.numel():   # (the norm below adds them row by row)
+            raise RuntimeError(f"attention gave {tuple(a.shape)} for {tuple(x.shape)}")
         x1_dtype = torch.promote_types(x.dtype, a.dtype)
         res = x.reshape(-1, C).to(torch.float32, copy=True)   # becomes x + a (a fresh copy)
         h = torch.empty_like(res)

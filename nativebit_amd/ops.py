@@ -18,7 +18,11 @@ _DT = {torch.float32: _lib.NB_F32, torch.bfloat16: _lib.NB_BF16}
 
 def _stream(t: torch.Tensor) -> int:
     """torch's current stream on t's device, as the ABI's hipStream_t (the raw
-    handle: torch.cuda.current_stream builds a Stream object, 2 us a call)."""
+    handle: torch.cuda.current_stream builds a Stream object, 2 us a call).
+    It refuses host tensors as current_stream does (the raw call takes device
+    -1 for the current one, and a kernel would read host addresses)."""
+    if not t.is_cuda:
+        raise ValueError(f"Expected a cuda device, but got: {t.device}")
     return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 

@@ -132,3 +132,40 @@ def test_kv_cache_shapes_and_layout():
         M._cache_storage(k.half(), v, 2, 4, 16)
     with pytest.raises(ValueError, match="positions"):
         M._cache_storage(k, torch.zeros(2, 4, 12, 16), 2, 4, 16)
+
+
+class _Fixed(torch.nn.Module):
+    """A linear of a wrong width: (B, T, in) -> (B, T, out) zeros."""
+
+    def __init__(self, out_f):
+        super().__init__()
+        self.out_f = out_f
+
+    def forward(self, x):
+        return torch.zeros(*x.shape[:-1], self.out_f)
+
+
+def test_host_tensors_and_mismatched_products_raise():
+    """The calls that hand raw addresses to kernels refuse host tensors
+    (torch.cuda.current_stream's error), gate and up outputs that differ in
+    shape (the product kernel walks both by one count), and an attention
+    output that the residual add cannot take row by row."""
+    from nativebit_amd.ops import _stream
+    with pytest.raises(ValueError, match="Expected a cuda device"):
+        _stream(torch.zeros(4))
+    with pytest.raises(ValueError, match="Expected a cuda device"):
+        M.RMSNorm(8)(torch.zeros(2, 8))
+    widths = iter((96, 48, 64))
+    ffn = M.SwiGLU(64, 96, lambda n, k: _Fixed(next(widths)))
+    with pytest.raises(RuntimeError, match="gate .*96.* up .*48"):
+        ffn(torch.zeros(1, 2, 64))
+
+    blk = M.TransformerBlock(64, 4, 96, 16, lambda n, k: _Fixed(n))
+    blk.ln1 = torch.nn.Identity()
+
+    class Narrow(torch.nn.Module):
+        def forward(self, x, kv_cache=None, pos_offset=0):
+            return x[..., :32], None
+    blk.attn = Narrow()
+    with pytest.raises(RuntimeError, match="attention gave"):
+        blk(torch.zeros(1, 2, 64))
