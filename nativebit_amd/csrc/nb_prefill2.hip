@@ -343,46 +343,61 @@ __global__ __launch_bounds__(64 * WAVES) void prefill2_kernel(Prefill2Args a) {
         if (step + 1 < nsteps) load_x(step + 1, cur ^ 1);
         const unsigned char* xt = smem + cur * kStage;
         const unsigned char* wt = xt + kXBytes;
-        auto read_w = [&](int c, u32x4_t (&av)[TI]) {
-#pragma unroll
-            for (int i = 0; i < TI; ++i)
-                av[i] = *reinterpret_cast<const u32x4_t*>(wt + swz(wn * WN + i * 16 + fr, c + fq));
+        // The fragment reads and MFMAs are written out where they are used:
+        // through helpers that take the fragment arrays by reference the
+        // compiler puts all twelve reads before the first MFMA of a half step
+        // (13824 x 2560 at M = 2048 173 us against 171).
+        auto w_frag = [&](int i, int c) {   // 16-byte chunk c of the wave's W rows
+            return *reinterpret_cast<const u32x4_t*>(wt + swz(wn * WN + i * 16 + fr, c));
         };
-        auto read_x = [&](int c, u32x4_t (&bv)[TJ]) {
-#pragma unroll
-            for (int j = 0; j < TJ; ++j)
-                bv[j] = *reinterpret_cast<const u32x4_t*>(xt + swz(wm * WM + j * 16 + fr, c + fq));
+        auto x_frag = [&](int j, int c) {
+            return *reinterpret_cast<const u32x4_t*>(xt + swz(wm * WM + j * 16 + fr, c));
         };
-        auto mfma_all = [&](const u32x4_t (&av)[TI], const u32x4_t (&bv)[TJ]) {
-#pragma unroll
-            for (int i = 0; i < TI; ++i)
-#pragma unroll
-                for (int j = 0; j < TJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf16x8_t, av[i]), __builtin_bit_cast(bf16x8_t, bv[j]),
-                        acc[i][j], 0, 0, 0);
+        auto mfma = [&](u32x4_t w, u32x4_t x, f32x4_t& sum) {
+            sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w),
+                                                          __builtin_bit_cast(bf16x8_t, x), sum, 0,
+                                                          0, 0);
         };
         if constexpr (kSplit) {
-            u32x4_t wv[TI], xv[TJ];
-            read_w(0, wv);
-            read_x(0, xv);
-            mfma_all(wv, xv);
-            u32x4_t wlo[TI];
-            read_w(4, wlo);
+            const int ch = fq, cl = 4 + fq;
+            u32x4_t wv[TI], xv[TJ], wlo[TI], xlo[TJ];
+#pragma unroll
+            for (int i = 0; i < TI; ++i) wv[i] = w_frag(i, ch);
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) xv[j] = x_frag(j, ch);
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) mfma(wv[i], xv[j], acc[i][j]);
+#pragma unroll
+            for (int i = 0; i < TI; ++i) wlo[i] = w_frag(i, cl);
             if (step + 1 < nsteps) store_w(cur ^ 1, next);
-            mfma_all(wlo, xv);
-            read_x(4, xv);
-            mfma_all(wv, xv);
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) mfma(wlo[i], xv[j], acc[i][j]);
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) xlo[j] = x_frag(j, cl);
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) mfma(wv[i], xlo[j], acc[i][j]);
         } else {
-            // 32 of the step's 64 K, then the other 32
-            u32x4_t av[TI], bv[TJ];
-            read_w(0, av);
-            read_x(0, bv);
-            mfma_all(av, bv);
+            auto half_step = [&](int half) {   // 32 of the step's 64 K
+                const int c = half * 4 + fq;
+                u32x4_t av[TI], bv[TJ];
+#pragma unroll
+                for (int i = 0; i < TI; ++i) av[i] = w_frag(i, c);
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) bv[j] = x_frag(j, c);
+#pragma unroll
+                for (int i = 0; i < TI; ++i)
+#pragma unroll
+                    for (int j = 0; j < TJ; ++j) mfma(av[i], bv[j], acc[i][j]);
+            };
+            half_step(0);
             if (step + 1 < nsteps) store_w(cur ^ 1, next);
-            read_w(4, av);
-            read_x(4, bv);
-            mfma_all(av, bv);
+            half_step(1);
         }
         // the next X slice (direct-to-LDS, not tracked by the compiler) must
         // be in LDS before the barrier; the W loads of step + 2, issued
