@@ -126,6 +126,9 @@ int nb_gemm_prefill(const void* x, int64_t ldx, const uint8_t* packed, const flo
  *           of the rest of this interface.
  */
 int64_t nb_gemm_prefill_split_ws_bytes(int M, int N, int K);
+/* The workspace with which nb_gemm_prefill_split runs its fastest plan (at
+ * least nb_gemm_prefill_split_ws_bytes; more is not used). */
+int64_t nb_gemm_prefill_split_best_ws_bytes(int M, int N, int K);
 int nb_gemm_prefill_split(const void* x, int64_t ldx, const uint8_t* packed,
                           const float* codebook, void* y, int y_dtype, int64_t ldy, int M, int N,
                           int K, void* workspace, int64_t ws_bytes, void* stream);
@@ -148,6 +151,9 @@ int nb_gemm_prefill_split(const void* x, int64_t ldx, const uint8_t* packed,
  *           nativebit/inference.py:42-46), without the per-call W.
  */
 int64_t nb_gemm_prefill_f32_ws_bytes(int M, int N, int K);
+/* The workspace with which nb_gemm_prefill_f32 runs its fastest plan (at
+ * least nb_gemm_prefill_f32_ws_bytes). */
+int64_t nb_gemm_prefill_f32_best_ws_bytes(int M, int N, int K);
 int nb_gemm_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed,
                         const float* codebook, float* y, int64_t ldy, int M, int N, int K,
                         void* workspace, int64_t ws_bytes, void* stream);

@@ -949,9 +949,18 @@ extern "C" int nb_gemm_prefill_split(const void* x, int64_t ldx, const uint8_t* 
                     (long long)need);
     }
     if (dev_st) return dev_st;
-    return launch_prefill2(x, ldx, packed, codebook, y, y_dtype, ldy, M, N, K,
-                           need > 0 ? workspace : nullptr, ws_bytes,
+    return launch_prefill2(x, ldx, packed, codebook, y, y_dtype, ldy, M, N, K, workspace, ws_bytes,
                            static_cast<hipStream_t>(stream));
+}
+
+extern "C" int64_t nb_gemm_prefill_split_best_ws_bytes(int M, int N, int K) {
+    if (ensure_device() != NB_OK) g_last_error[0] = '\0';
+    return prefill_split_best_bytes(M, N, K);
+}
+
+extern "C" int64_t nb_gemm_prefill_f32_best_ws_bytes(int M, int N, int K) {
+    if (ensure_device() != NB_OK) g_last_error[0] = '\0';
+    return prefill_f32_best_bytes(M, N, K);
 }
 
 extern "C" int64_t nb_gemm_prefill_f32_ws_bytes(int M, int N, int K) {
@@ -982,7 +991,7 @@ extern "C" int nb_gemm_prefill_f32(const float* x, int64_t ldx, const uint8_t* p
                     (long long)need);
     }
     if (dev_st) return dev_st;
-    return launch_prefill_f32(x, ldx, packed, codebook, y, ldy, M, N, K, workspace,
+    return launch_prefill_f32(x, ldx, packed, codebook, y, ldy, M, N, K, workspace, ws_bytes,
                               static_cast<hipStream_t>(stream));
 }
 

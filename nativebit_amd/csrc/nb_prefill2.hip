@@ -207,8 +207,8 @@ struct WRegs {
 // rounded to bf16).  The fragments of a step then feed three MFMAs instead of
 // two, so this form reads less LDS per MFMA than the bf16 one.  Measured
 // against three passes of the bf16 kernel that added to y (and a residual
-// codebook made per call): 7680 x 2560 at M = 128 / 500 / 2048 37 / 84 / 236 us
-// (72 / 129 / 286), 2560 x 6912 40 / 73 / 245 us (78 / 145 / 313), the same
+// codebook made per call): 7680 x 2560 at M = 128 / 500 / 2048 34 / 71 / 221 us
+// (72 / 129 / 286), 2560 x 6912 34 / 68 / 227 us (78 / 145 / 313), the same
 // 4.3e-6 from fp64.
 template <int BM, int BN, int WAVES, bool kSplit>
 __global__ __launch_bounds__(64 * WAVES) void prefill2_kernel(Prefill2Args a) {
@@ -472,10 +472,11 @@ constexpr TileCost kBf16Tiles[] = {{256, 256, 1, 5.9f, {1.71f}},
                                    {256, 128, 1, 3.4f, {1.09f}},
                                    {128, 128, 2, 3.3f, {0.74f, 1.15f}},
                                    {64, 128, 3, 2.7f, {0.57f, 0.91f, 1.42f}}};
-// three products (two steps of 32 per 64 of K; they spill at 256 x 256)
-constexpr TileCost kF32Tiles[] = {{256, 128, 1, 0.4f, {2.55f}},
-                                  {128, 128, 2, 1.2f, {1.76f, 3.34f}},
-                                  {64, 128, 3, 1.2f, {1.34f, 2.00f, 3.03f}}};
+// three products (two steps of 32 per 64 of K; they spill at 256 x 256);
+// fitted to 283 plans (four layer shapes, M = 17 .. 2048, mean error 3.4 %)
+constexpr TileCost kF32Tiles[] = {{256, 128, 1, 0.0f, {2.63f}},
+                                  {128, 128, 2, 0.9f, {1.73f, 2.65f}},
+                                  {64, 128, 2, 2.2f, {1.25f, 1.88f}}};
 constexpr int kMinSplitSteps = 4;
 
 inline int64_t grid_of(int M, int N, int bm, int bn) {
@@ -483,13 +484,23 @@ inline int64_t grid_of(int M, int N, int bm, int bn) {
 }
 
 // Estimated time of S K ranges per tile: the busiest CU takes
-// ceil(workgroups / CUs) of them, `resident` at a time; S > 1 adds the
-// reduction launch (r0) and the partial products' write and read (rb a MB).
+// ceil(workgroups / CUs) of them, `resident` at a time (kTail: what is left
+// over for the last round at the cost of that many, as the fp32 costs were
+// fitted); S > 1 adds the reduction launch (r0) and the partial products'
+// write and read (rb a MB).
+template <bool kTail>
 float plan_time(const TileCost& c, int S, int M, int N, int K, int64_t cus, float r0, float rb) {
     const int64_t per = (grid_of(M, N, c.BM, c.BN) * S + cus - 1) / cus;
-    const int64_t conc = std::min<int64_t>(per, c.resident);
-    const float rounds = (float)((per + conc - 1) / conc);
-    const float t = rounds * (c.start + (float)((K / kBK + S - 1) / S) * c.step[conc - 1]);
+    const float steps = (float)((K / kBK + S - 1) / S);
+    float t;
+    if (kTail) {
+        t = (float)(per / c.resident) * (c.start + steps * c.step[c.resident - 1]);
+        const int64_t rest = per % c.resident;
+        if (rest) t += c.start + steps * c.step[rest - 1];
+    } else {
+        const int64_t conc = std::min<int64_t>(per, c.resident);
+        t = (float)((per + conc - 1) / conc) * (c.start + steps * c.step[conc - 1]);
+    }
     return S > 1 ? t + r0 + rb * 4e-6f * (float)S * (float)M * (float)N : t;
 }
 
@@ -504,14 +515,18 @@ float plan_time(const TileCost& c, int S, int M, int N, int K, int64_t cus, floa
 // 24.0 -> 11.7 / 13.3 us, 1024 x 4096 35 -> 12 us, 5000 x 1024 at M = 300 22 ->
 // 14.6 us, 2560 x 6912 at M = 700 55 -> 47 us; the sizes that the thresholds
 // were tuned on keep their plans or ones as fast.
-PrefillPlan prefill_plan(int M, int N, int K, bool allow_split) {
+// A grid that reaches 0.6 of the CUs is split too where the caller's
+// workspace (ws_bytes, beyond what prefill_split_bytes asks for) holds the
+// partial products and the estimate is a tenth less: 2560 x 6912 at M = 1024 88
+// -> 56 us (three ranges of 256 x 128).
+PrefillPlan prefill_plan(int M, int N, int K, bool allow_split, int64_t ws_bytes) {
     const int64_t cus = device_cu_count();
     const int nsteps = K / kBK;
     const int64_t limit = 4 * ((int64_t)N * K / 128 * 80);
     PrefillPlan best = {64, 128, 1};
     float best_t = INFINITY;
     auto offer = [&](const TileCost& c, int S) {
-        const float t = plan_time(c, S, M, N, K, cus, 5.5f, 0.30f);
+        const float t = plan_time<false>(c, S, M, N, K, cus, 5.5f, 0.30f);
         if (t < best_t) {
             best_t = t;
             best = {c.BM, c.BN, S};
@@ -530,19 +545,24 @@ PrefillPlan prefill_plan(int M, int N, int K, bool allow_split) {
             const int S = (int)std::min<int64_t>(cus / g, nsteps / 32);
             if (S >= 2 && g * S > full) offer(kBf16Tiles[0], S);
         }
-        return best;
+        if (best.S > 1) return best;
+        best_t *= 0.9f;
+    } else {
+        best_t *= 1.1f;   // (the estimates' error: split where it costs about the same)
     }
-    best_t *= 1.1f;   // (the estimates' error: split where it costs about the same)
+    const int64_t most = full ? std::min(limit, ws_bytes) : limit;
     for (const TileCost& c : kBf16Tiles) {
         for (int S = 2; S <= 8 && nsteps / S >= kMinSplitSteps; ++S) {
-            if ((int64_t)S * M * N * 4 <= limit) offer(c, S);
+            if ((int64_t)S * M * N * 4 <= most) offer(c, S);
         }
     }
     return best;
 }
 
 // fp32 activations: any number of K ranges up to 16 whose partial products
-// fit `limit` bytes (2560 x 2560 at M = 64 56 -> 22 us).
+// fit `limit` bytes (2560 x 2560 at M = 64 56 -> 22 us; 7680 x 2560 at M = 500
+// in two ranges of 256 x 128 79 -> 71 us).  Unsplit plans take 1-9 % longer
+// than estimated.
 PrefillPlan prefill_f32_plan(int M, int N, int K, int64_t limit) {
     const int64_t cus = device_cu_count();
     PrefillPlan best = {64, 128, 1};
@@ -550,7 +570,7 @@ PrefillPlan prefill_f32_plan(int M, int N, int K, int64_t limit) {
     for (const TileCost& c : kF32Tiles) {
         for (int S = 1; S <= 16; ++S) {
             if (S > 1 && (K / kBK / S < kMinSplitSteps || (int64_t)S * M * N * 4 > limit)) break;
-            const float t = plan_time(c, S, M, N, K, cus, 8.7f, 0.43f);
+            const float t = plan_time<true>(c, S, M, N, K, cus, 8.75f, 0.312f) * (S > 1 ? 1.f : 1.06f);
             if (t < best_t) {
                 best_t = t;
                 best = {c.BM, c.BN, S};
@@ -604,8 +624,14 @@ inline int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
 int64_t prefill_split_bytes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
-    const PrefillPlan p = prefill_plan(M, N, K, true);
+    const PrefillPlan p = prefill_plan(M, N, K, true, 0);
     return p.S > 1 ? (int64_t)p.S * M * N * 4 : 0;
+}
+
+int64_t prefill_split_best_bytes(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
+    const PrefillPlan p = prefill_plan(M, N, K, true, INT64_MAX);
+    return std::max(p.S > 1 ? (int64_t)p.S * M * N * 4 : 0, prefill_split_bytes(M, N, K));
 }
 
 namespace {
@@ -647,8 +673,8 @@ int launch_tiles(Prefill2Args a, const PrefillPlan& p, void* workspace, hipStrea
 int launch_prefill2(const void* x, int64_t ldx, const uint8_t* packed, const float* codebook,
                     void* y, int y_dtype, int64_t ldy, int M, int N, int K, void* workspace,
                     int64_t ws_bytes, hipStream_t stream) {
-    PrefillPlan p = prefill_plan(M, N, K, workspace != nullptr);
-    if (p.S > 1 && ws_bytes < (int64_t)p.S * M * N * 4) p = prefill_plan(M, N, K, false);
+    PrefillPlan p = prefill_plan(M, N, K, workspace != nullptr, ws_bytes);
+    if (p.S > 1 && ws_bytes < (int64_t)p.S * M * N * 4) p = prefill_plan(M, N, K, false, 0);
     return launch_tiles<false>({static_cast<const uint16_t*>(x), ldx, packed, codebook, y, ldy,
                                 y_dtype, M, N, K, 1, nullptr}, p, workspace, stream);
 }
@@ -663,9 +689,17 @@ int64_t prefill_f32_bytes(int M, int N, int K) {
     return 2 * xb + cb + prefill_split_bytes(M, N, K);
 }
 
+int64_t prefill_f32_best_bytes(int M, int N, int K) {
+    const int64_t least = prefill_f32_bytes(M, N, K);
+    if (least == 0) return 0;
+    const PrefillPlan p = prefill_f32_plan(M, N, K, 128LL << 20);
+    const int64_t part = p.S > 1 ? (int64_t)p.S * M * N * 4 : 0;
+    return std::max(least, align256((int64_t)M * K * 4) + part);
+}
+
 int launch_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed, const float* codebook,
                        float* y, int64_t ldy, int M, int N, int K, void* workspace,
-                       hipStream_t stream) {
+                       int64_t ws_bytes, hipStream_t stream) {
     GemvArgs rows;
     rows.x = x;
     rows.x_dtype = NB_F32;
@@ -699,7 +733,7 @@ int launch_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed, const
     if (st) return st;
     return launch_tiles<true>({xs, 2 * (int64_t)K, packed, codebook, y, ldy, NB_F32, M, N, K, 1,
                                nullptr},
-                              prefill_f32_plan(M, N, K, prefill_f32_bytes(M, N, K) - xbytes),
+                              prefill_f32_plan(M, N, K, ws_bytes - xbytes),
                               w + xbytes, stream);
 }
 

@@ -405,7 +405,7 @@ def gemm_prefill(x: torch.Tensor, packed: torch.Tensor, codebook: torch.Tensor, 
         raise ValueError(f"unknown prefill path {path!r}")
     lib = _lib.load()
     if path == "auto":
-        nbytes = int(lib.nb_gemm_prefill_split_ws_bytes(M, N, K))
+        nbytes = int(lib.nb_gemm_prefill_split_best_ws_bytes(M, N, K))
         ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
         _lib.check(lib.nb_gemm_prefill_split(
             x.data_ptr(), x.stride(0), packed.data_ptr(), codebook.data_ptr(), out.data_ptr(),
@@ -443,7 +443,7 @@ def gemm_prefill_f32(x: torch.Tensor, packed: torch.Tensor, codebook: torch.Tens
     elif out.shape != (M, N) or out.dtype != torch.float32 or out.stride(1) != 1:
         raise ValueError("out must be (M, N) float32, row-contiguous")
     lib = _lib.load()
-    nbytes = int(lib.nb_gemm_prefill_f32_ws_bytes(M, N, K))
+    nbytes = int(lib.nb_gemm_prefill_f32_best_ws_bytes(M, N, K))
     ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
     _lib.check(lib.nb_gemm_prefill_f32(
         x.data_ptr(), x.stride(0), packed.data_ptr(), codebook.data_ptr(), out.data_ptr(),

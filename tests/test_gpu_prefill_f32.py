@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from nativebit_amd import ops
+from nativebit_amd import _lib, ops
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -46,3 +46,42 @@ def test_f32_strided_rows(dev, pad):
     """Rows of x with and without 16-byte alignment."""
     assert _case(dev, 200, 3000, 1024, pad).max() <= 1.0
     assert _case(dev, 20, 300, 256, pad).max() <= 1.0
+
+
+@pytest.mark.parametrize("f32", [True, False])
+@pytest.mark.parametrize("m,n,k", [
+    (500, 7680, 2560), (290, 6912, 1280), (1000, 2560, 6912), (257, 2561, 4096), (40, 128, 384)])
+def test_plans_of_both_workspaces(dev, f32, m, n, k):
+    """The fastest plan (the workspace of *_best_ws_bytes) and the one of
+    *_ws_bytes write only their workspace and y.  fp32: the bound above; bf16:
+    exact products of bf16 values in fp32 sums, (K / 32 + 40) 2^-24 sum |x w|."""
+    print(f"[case] prefill plans {m}x{n}x{k} f32={f32}", flush=True)
+    lib = _lib.load()
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    idx = torch.randint(0, 8, (n * k,), generator=g, device=dev, dtype=torch.uint8)
+    cb = torch.randn(n * k // 128, 8, generator=g, device=dev) * 0.02
+    packed = ops.pack(idx, 3)
+    x = torch.randn(m, k, generator=g, device=dev)
+    if not f32:
+        x, cb = x.bfloat16(), cb.bfloat16().float()
+    w = cb.double().gather(1, idx.view(-1, 128).long()).view(n, k)
+    ref, size = x.double() @ w.T, x.double().abs() @ w.T.abs()
+    bound = (3 * 2.0 ** -18 + (3 * k / 32 + 48) * 2.0 ** -24 if f32 else (k / 32 + 40) * 2.0 ** -24) * size
+    name = "nb_gemm_prefill_f32" if f32 else "nb_gemm_prefill_split"
+    least = getattr(lib, name + "_ws_bytes")(m, n, k)
+    best = getattr(lib, name + "_best_ws_bytes")(m, n, k)
+    assert best >= least
+    for nbytes in {least, best}:
+        ws = torch.full((nbytes + 4096,), 0xff, dtype=torch.uint8, device=dev)
+        y = torch.empty(m + 1, n, device=dev)
+        y[m] = 7.0
+        args = (m, n, k, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+        if f32:
+            st = lib.nb_gemm_prefill_f32(x.data_ptr(), k, packed.data_ptr(), cb.data_ptr(),
+                                         y.data_ptr(), n, *args)
+        else:
+            st = lib.nb_gemm_prefill_split(x.data_ptr(), k, packed.data_ptr(), cb.data_ptr(),
+                                           y.data_ptr(), _lib.NB_F32, n, *args)
+        _lib.check(st)
+        assert (ws[nbytes:] == 0xff).all() and (y[m] == 7.0).all()
+        assert ((y[:m].double() - ref).abs() <= bound).all()
