@@ -52,6 +52,7 @@ def bits_for_entries(n_entries: int) -> int:
 
 def packed_nbytes(count: int, bits: int) -> int:
     """Bytes of a packed stream (nb_packed_nbytes)."""
+    count, bits = int(count), int(bits)
     if not 1 <= bits <= 8 or count < 0:
         return 0
     return -(-count // 8) * 3 if bits == 3 else (count * bits + 7) // 8

@@ -169,3 +169,16 @@ def test_host_tensors_and_mismatched_products_raise():
     blk.attn = Narrow()
     with pytest.raises(RuntimeError, match="attention gave"):
         blk(torch.zeros(1, 2, 64))
+
+
+def test_packed_nbytes_equals_the_library():
+    """ops.packed_nbytes without the call: nb_packed_nbytes' values, as whole
+    numbers also for float counts (which int() truncates)."""
+    from nativebit_amd import _lib, ops
+    lib = _lib.load()
+    for bits in range(-1, 10):
+        for count in (-9, -1, 0, 1, 7, 8, 9, 31, 32, 33, 127, 6912 * 2560, 2 ** 33 + 5):
+            assert ops.packed_nbytes(count, bits) == lib.nb_packed_nbytes(count, bits), (count, bits)
+    for count in (9.0, 9.5):
+        got = ops.packed_nbytes(count, 3.0)
+        assert isinstance(got, int) and got == lib.nb_packed_nbytes(9, 3)
