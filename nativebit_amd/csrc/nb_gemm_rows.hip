@@ -22,7 +22,7 @@
 //
 // Split: a workgroup owns 16 output rows; its waves split K in whole
 // 128-column units and add their accumulators through LDS once at the end,
-// in wave order (deterministic).  Activations are read from global memory
+// in wave order and fp64 (deterministic).  Activations are read from global memory
 // (the L2 holds them: at most 64 rows) straight into registers, a group of 8
 // columns at a time, the next groups requested as the current one is used;
 // the next unit's index bytes and block entries are requested before the
@@ -33,8 +33,10 @@
 // gemv_generic_kernel took 157 / 160 / 60.  What is left at M = 8, from copies
 // with parts taken out: 10 us the weights' loads and MFMAs, 1.2 the lookups,
 // 2 the activations (5.4 at M = 16: a lane's 32 columns are a cache line of
-// their own).  fp64 errors 1.2-1.4e-7, the one-row kernel's; four short
-// accumulators a unit keep them there (one chain a wave: 2-3e-7).
+// their own).  fp64 errors at M <= 16 8.0-9.3e-8 from 512 x 512 to 16384 x
+// 2560 (gemv_generic_kernel 8.5e-8-1.3e-7): accumulators of 8 products, added
+// pairwise; with ones of 32 products 1.2-1.4e-7 at up to 1 % less time, with
+// one chain a wave 2-3e-7.
 //
 // Formats: 2/3/4-bit with 2^bits entries, BS 64/128/256, K % 128 == 0 and
 // K % BS == 0.
@@ -80,7 +82,9 @@ template <int BITS, int BS, int TM>
 __global__ __launch_bounds__(64 * max_waves(TM)) void gemm_rows_f32_kernel(RowsArgs a) {
     constexpr int NE = 1 << BITS;
     constexpr uint32_t kTab = NE * 256;          // a wave's entry-major table
-    constexpr int D = TM == 1 ? 4 : 2;           // 8-column groups of x in registers
+    // 8-column groups of x in registers (four beside 16 entries spill: 2000 x
+    // 8192 at M = 5 27.0 us against 22.6)
+    constexpr int D = TM == 1 && BITS < 4 ? 4 : 2;
     extern __shared__ __align__(16) unsigned char smem[];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nwaves = blockDim.x >> 6;
     const int r = lane & 15, g = lane >> 4;
@@ -139,14 +143,12 @@ __global__ __launch_bounds__(64 * max_waves(TM)) void gemm_rows_f32_kernel(RowsA
 #pragma unroll
             for (int i = 0; i < BITS; ++i) d[i] = w.d[i];
             if (u + 1 < u1) load_unit(u + 1, w);
-            // four accumulators a unit, added to the wave's sum: short
-            // chains, so the sums are as close to fp64 as a wave-wide tree's
-            f32x4_t acc[TM][4];
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-            }
+            // four accumulators, of a group of 8 columns for up to 16 rows (8
+            // products each), of the unit beyond (32), added pairwise and
+            // then to the wave's sum
+            constexpr bool kShort = TM == 1;
+            const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+            f32x4_t acc[TM][4], half[2];
             auto group = [&](auto qc) {
                 constexpr int q = decltype(qc)::value;
                 float wv[8];
@@ -157,8 +159,13 @@ __global__ __launch_bounds__(64 * max_waves(TM)) void gemm_rows_f32_kernel(RowsA
 #pragma unroll
                     for (int i = 0; i < TM; ++i) {
                         acc[i][j & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                            wv[j], x[i][j >> 2][j & 3], acc[i][j & 3], 0, 0, 0);
+                            wv[j], x[i][j >> 2][j & 3],
+                            j < 4 && (kShort || q == 0) ? zero : acc[i][j & 3], 0, 0, 0);
                     }
+                }
+                if constexpr (kShort) {
+                    const f32x4_t p = (acc[0][0] + acc[0][1]) + (acc[0][2] + acc[0][3]);
+                    half[q / 2] = q % 2 ? half[q / 2] + p : p;
                 }
                 // the group D ahead, into the registers just used
                 if constexpr (q + D < 4) {
@@ -173,13 +180,14 @@ __global__ __launch_bounds__(64 * max_waves(TM)) void gemm_rows_f32_kernel(RowsA
             group(std::integral_constant<int, 3>{});
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
-                sum[i] += (acc[i][0] + acc[i][1]) + (acc[i][2] + acc[i][3]);
+                sum[i] += kShort ? half[0] + half[1]
+                                 : (acc[i][0] + acc[i][1]) + (acc[i][2] + acc[i][3]);
             }
         }
     }
 
     // lane (r, g) of tile i holds W rows 4 g + v of activation row 16 i + r:
-    // the waves' sums in wave order
+    // the waves' sums in wave order, in fp64 (rounded once)
     float* red = reinterpret_cast<float*>(smem);
     __syncthreads();   // the tables are no longer read
 #pragma unroll
@@ -191,8 +199,9 @@ __global__ __launch_bounds__(64 * max_waves(TM)) void gemm_rows_f32_kernel(RowsA
     for (int e = t; e < TM * 256; e += blockDim.x) {
         const int m = e >> 4, n = e & 15;
         if (m >= a.M || row0 + n >= a.N) continue;
-        float s = 0.f;
-        for (int w = 0; w < nwaves; ++w) s += red[(w * TM * 16 + m) * 20 + n];
+        double sd = 0.0;
+        for (int w = 0; w < nwaves; ++w) sd += red[(w * TM * 16 + m) * 20 + n];
+        const float s = (float)sd;
         const int64_t o = (int64_t)m * a.ldy + row0 + n;
         if (a.y_dtype == NB_BF16) {
             static_cast<bf16_bits*>(a.y)[o] = f32_to_bf16_rne(s);
