@@ -84,9 +84,8 @@ class PackedLinear(torch.nn.Module):
             # (.to(tl.float32), triton_kernel.py:46, 174-183)
             x_flat = x_flat.to(torch.float32)
         if M <= MAX_GEMV_ROWS:
-            buffers = self._buffers   # (nn.Module's attribute lookup, 0.3 us each)
-            y = ops.gemv(x_flat, buffers["packed_indices"], buffers["codebook"], N, K,
-                         bits=self.bits, block_size=self.block_size, out_dtype=self.out_dtype)
+            y = ops.gemv(x_flat, self.packed_indices, self.codebook, N, K, bits=self.bits,
+                         block_size=self.block_size, out_dtype=self.out_dtype)
         elif x_flat.dtype == torch.bfloat16 and self._standard():
             # the bf16 batched form (eval_ppl.py:149-174): the packed MFMA kernels
             y = ops.gemm_prefill(x_flat, self.packed_indices, self.codebook, N, K,
