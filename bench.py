@@ -499,7 +499,7 @@ PREFILL_SHAPES = (("qkv", 7680, 2560), ("o", 2560, 2560), ("gate|up", 13824, 256
 def bench_prefill(dev, random_weights=False):
     """Config 4a: prefill-sized contraction with the packed weights.
 
-    The value is nb_gemm_prefill_split (ops.gemm_prefill's default): the
+    The value is nb_gemm_prefill_split_best (ops.gemm_prefill's default): the
     hand-written MFMA kernels that dequantize the 3-bit stream into LDS
     tiles, split over K ranges where one launch's tile grid would leave CUs
     idle; beside it the one-launch kernel (nb_gemm_prefill) and, for
@@ -550,7 +550,7 @@ def bench_prefill(dev, random_weights=False):
                                            [graph_calls_time(f) for f in fns])]
             ms, ms_one, ms_blas, ms_ref, ms_f32, ms_f32_ref = t
             fl = 2 * M * N * K
-            ws = int(_lib.load().nb_gemm_prefill_split_ws_bytes(M, N, K))
+            ws = int(_lib.load().nb_gemm_prefill_split_best_ws_bytes(M, N, K))
             per[n] = {"us": round(ms * 1e3, 1), "TFLOP_s": round(fl / ms / 1e9, 1),
                       "k_split_partials_MiB": round(ws / 2**20, 2),
                       "one_launch_us": round(ms_one * 1e3, 1),
@@ -575,7 +575,7 @@ def bench_prefill(dev, random_weights=False):
                         "f32_x_TFLOP_s": round(tot_fl / f32_ms / 1e9, 1),
                         "f32_x_gather_then_torch_f32_layer_us": round(f32_ref_ms * 1e3, 1),
                         "per_matmul": per}
-    out["note"] = ("us / TFLOP_s: nb_gemm_prefill_split, the hand-written MFMA kernels that "
+    out["note"] = ("us / TFLOP_s: nb_gemm_prefill_split_best, the hand-written MFMA kernels that "
                    "read the 3-bit stream and codebooks and dequantize into LDS (bf16 operands, "
                    "fp32 accumulation, bf16 y), with a K split (fp32 partials in a workspace, "
                    "one reduction launch) where the tile grid would leave CUs idle "
@@ -587,9 +587,9 @@ def bench_prefill(dev, random_weights=False):
                    "(hipBLASLt), the expansion inside the timed call, "
                    "torch_dense_bf16 = torch.matmul on an already-unpacked bf16 weight (the "
                    "reference's path also unpacks and gathers W on every call, "
-                   "triton_kernel.py:258-275); f32_x = nb_gemm_prefill_f32 for fp32 activations "
-                   "against the exact fp32 weights (three bf16 MFMA passes over the hi / lo parts "
-                   "of x and W, fp32-level products), beside f32_x_gather_then_torch_f32 = the "
+                   "triton_kernel.py:258-275); f32_x = nb_gemm_prefill_f32_best for fp32 "
+                   "activations against the exact fp32 weights (three bf16 MFMA products a step "
+                   "over the hi / lo parts of x and W, fp32-level products), beside f32_x_gather_then_torch_f32 = the "
                    "reference's fp32 batched branch on the GPU (nb_dequant to fp32 W, then "
                    "torch.matmul in fp32)")
     return out

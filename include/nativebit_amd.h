@@ -126,12 +126,13 @@ int nb_gemm_prefill(const void* x, int64_t ldx, const uint8_t* packed, const flo
  *           of the rest of this interface.
  */
 int64_t nb_gemm_prefill_split_ws_bytes(int M, int N, int K);
-/* The workspace with which nb_gemm_prefill_split runs its fastest plan (at
- * least nb_gemm_prefill_split_ws_bytes; more is not used). */
-int64_t nb_gemm_prefill_split_best_ws_bytes(int M, int N, int K);
 int nb_gemm_prefill_split(const void* x, int64_t ldx, const uint8_t* packed,
                           const float* codebook, void* y, int y_dtype, int64_t ldy, int M, int N,
                           int K, void* workspace, int64_t ws_bytes, void* stream);
+int64_t nb_gemm_prefill_split_best_ws_bytes(int M, int N, int K);
+int nb_gemm_prefill_split_best(const void* x, int64_t ldx, const uint8_t* packed,
+                               const float* codebook, void* y, int y_dtype, int64_t ldy, int M,
+                               int N, int K, void* workspace, int64_t ws_bytes, void* stream);
 
 /*
  * The same contraction for fp32 activations against the exact fp32 codebook
@@ -144,19 +145,25 @@ int nb_gemm_prefill_split(const void* x, int64_t ldx, const uint8_t* packed,
  * against 2^-24 for an fp32 product; few rows of a small layer run on fp32
  * MFMAs with the exact products.  W is never materialised.  The workspace
  * needs nb_gemm_prefill_f32_ws_bytes(M, N, K) bytes, 256-byte aligned (the
- * bf16 parts of x, the K-split partial products), contents clobbered.
- * Deterministic.
+ * bf16 parts of x, the K-split partial products), which are clobbered; bytes
+ * beyond them are not touched.  nb_gemm_prefill_f32_best is the same call
+ * with the plan that is fastest with up to 128 MiB of partial products (or
+ * what the least workspace holds of them, where that is more); its workspace
+ * needs nb_gemm_prefill_f32_best_ws_bytes(M, N, K) bytes.  The order of the
+ * fp32 sums follows from the entry point, M, N and K (few rows: also x's
+ * alignment), never from ws_bytes.  Deterministic.
  * Replaces: the batched branch of PackedLinear.forward for fp32 x
  *           (unpack + gather + x @ W.T, inference/triton_kernel.py:258-275;
  *           nativebit/inference.py:42-46), without the per-call W.
  */
 int64_t nb_gemm_prefill_f32_ws_bytes(int M, int N, int K);
-/* The workspace with which nb_gemm_prefill_f32 runs its fastest plan (at
- * least nb_gemm_prefill_f32_ws_bytes). */
-int64_t nb_gemm_prefill_f32_best_ws_bytes(int M, int N, int K);
 int nb_gemm_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed,
                         const float* codebook, float* y, int64_t ldy, int M, int N, int K,
                         void* workspace, int64_t ws_bytes, void* stream);
+int64_t nb_gemm_prefill_f32_best_ws_bytes(int M, int N, int K);
+int nb_gemm_prefill_f32_best(const float* x, int64_t ldx, const uint8_t* packed,
+                             const float* codebook, float* y, int64_t ldy, int M, int N, int K,
+                             void* workspace, int64_t ws_bytes, void* stream);
 
 /*
  * Unpack `count` indices of `bits` bits to one byte each.

@@ -920,21 +920,25 @@ extern "C" int nb_gemm_prefill(const void* x, int64_t ldx, const uint8_t* packed
     if (st || done) return st;
     st = ensure_device();
     if (st) return st;
-    return launch_prefill2(x, ldx, packed, codebook, y, y_dtype, ldy, M, N, K, nullptr, 0,
-                           static_cast<hipStream_t>(stream));
+    return launch_prefill2(x, ldx, packed, codebook, y, y_dtype, ldy, M, N, K, nullptr,
+                           PlanSpace::kNone, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int64_t nb_gemm_prefill_split_ws_bytes(int M, int N, int K) {
-    // without a usable device the plan assumes 256 CUs (and no error is left)
+namespace {
+// Workspace sizes without a usable device assume 256 CUs (and no error is
+// left).
+int64_t split_ws_bytes(int M, int N, int K, PlanSpace space) {
     if (ensure_device() != NB_OK) g_last_error[0] = '\0';
-    return prefill_split_bytes(M, N, K);
+    return prefill_split_bytes(M, N, K, space);
+}
+int64_t f32_ws_bytes(int M, int N, int K, PlanSpace space) {
+    if (ensure_device() != NB_OK) g_last_error[0] = '\0';
+    return prefill_f32_bytes(M, N, K, space);
 }
 
-extern "C" int nb_gemm_prefill_split(const void* x, int64_t ldx, const uint8_t* packed,
-                                     const float* codebook, void* y, int y_dtype, int64_t ldy,
-                                     int M, int N, int K, void* workspace, int64_t ws_bytes,
-                                     void* stream) {
-    const char* fn = "nb_gemm_prefill_split";
+int prefill_split(const char* fn, const void* x, int64_t ldx, const uint8_t* packed,
+                  const float* codebook, void* y, int y_dtype, int64_t ldy, int M, int N, int K,
+                  void* workspace, int64_t ws_bytes, PlanSpace space, void* stream) {
     bool done;
     int st = check_prefill(fn, x, ldx, packed, codebook, y, y_dtype, ldy, M, N, K, &done);
     if (st || done) return st;
@@ -943,34 +947,19 @@ extern "C" int nb_gemm_prefill_split(const void* x, int64_t ldx, const uint8_t* 
     // the size check comes before the device's status, so that it holds (for
     // 256 CUs) where there is no device
     const int dev_st = ensure_device();
-    const int64_t need = prefill_split_bytes(M, N, K);
+    const int64_t need = prefill_split_bytes(M, N, K, space);
     if (ws_bytes < need || (need > 0 && !workspace)) {
         return fail(NB_EINVAL, "%s: workspace of %lld bytes < %lld", fn, (long long)ws_bytes,
                     (long long)need);
     }
     if (dev_st) return dev_st;
-    return launch_prefill2(x, ldx, packed, codebook, y, y_dtype, ldy, M, N, K, workspace, ws_bytes,
+    return launch_prefill2(x, ldx, packed, codebook, y, y_dtype, ldy, M, N, K, workspace, space,
                            static_cast<hipStream_t>(stream));
 }
 
-extern "C" int64_t nb_gemm_prefill_split_best_ws_bytes(int M, int N, int K) {
-    if (ensure_device() != NB_OK) g_last_error[0] = '\0';
-    return prefill_split_best_bytes(M, N, K);
-}
-
-extern "C" int64_t nb_gemm_prefill_f32_best_ws_bytes(int M, int N, int K) {
-    if (ensure_device() != NB_OK) g_last_error[0] = '\0';
-    return prefill_f32_best_bytes(M, N, K);
-}
-
-extern "C" int64_t nb_gemm_prefill_f32_ws_bytes(int M, int N, int K) {
-    return prefill_f32_bytes(M, N, K);
-}
-
-extern "C" int nb_gemm_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed,
-                                   const float* codebook, float* y, int64_t ldy, int M, int N,
-                                   int K, void* workspace, int64_t ws_bytes, void* stream) {
-    const char* fn = "nb_gemm_prefill_f32";
+int prefill_f32(const char* fn, const float* x, int64_t ldx, const uint8_t* packed,
+                const float* codebook, float* y, int64_t ldy, int M, int N, int K, void* workspace,
+                int64_t ws_bytes, PlanSpace space, void* stream) {
     if (M < 0 || N < 0 || K < 0) return fail(NB_EINVAL, "%s: negative shape", fn);
     if (K % 128 != 0) return fail(NB_EUNSUPPORTED, "%s: K=%d not a multiple of 128", fn, K);
     if ((int64_t)N * (K / 128) >= (1LL << 31) || (int64_t)M * K >= (1LL << 40)) {
@@ -985,14 +974,61 @@ extern "C" int nb_gemm_prefill_f32(const float* x, int64_t ldx, const uint8_t* p
     if (!aligned(packed, 8) || !aligned(codebook, 16)) return fail(NB_EALIGN, "%s: packed 8- / codebook 16-byte alignment", fn);
     if (!aligned(workspace, 256)) return fail(NB_EALIGN, "%s: workspace not 256-byte aligned", fn);
     const int dev_st = ensure_device();
-    const int64_t need = prefill_f32_bytes(M, N, K);
+    const int64_t need = prefill_f32_bytes(M, N, K, space);
     if (ws_bytes < need) {
         return fail(NB_EINVAL, "%s: workspace of %lld bytes < %lld", fn, (long long)ws_bytes,
                     (long long)need);
     }
     if (dev_st) return dev_st;
-    return launch_prefill_f32(x, ldx, packed, codebook, y, ldy, M, N, K, workspace, ws_bytes,
+    return launch_prefill_f32(x, ldx, packed, codebook, y, ldy, M, N, K, workspace, space,
                               static_cast<hipStream_t>(stream));
+}
+}  // namespace
+
+extern "C" int64_t nb_gemm_prefill_split_ws_bytes(int M, int N, int K) {
+    return split_ws_bytes(M, N, K, PlanSpace::kLeast);
+}
+
+extern "C" int nb_gemm_prefill_split(const void* x, int64_t ldx, const uint8_t* packed,
+                                     const float* codebook, void* y, int y_dtype, int64_t ldy,
+                                     int M, int N, int K, void* workspace, int64_t ws_bytes,
+                                     void* stream) {
+    return prefill_split("nb_gemm_prefill_split", x, ldx, packed, codebook, y, y_dtype, ldy, M, N,
+                         K, workspace, ws_bytes, PlanSpace::kLeast, stream);
+}
+
+extern "C" int64_t nb_gemm_prefill_split_best_ws_bytes(int M, int N, int K) {
+    return split_ws_bytes(M, N, K, PlanSpace::kBest);
+}
+
+extern "C" int nb_gemm_prefill_split_best(const void* x, int64_t ldx, const uint8_t* packed,
+                                          const float* codebook, void* y, int y_dtype, int64_t ldy,
+                                          int M, int N, int K, void* workspace, int64_t ws_bytes,
+                                          void* stream) {
+    return prefill_split("nb_gemm_prefill_split_best", x, ldx, packed, codebook, y, y_dtype, ldy, M,
+                         N, K, workspace, ws_bytes, PlanSpace::kBest, stream);
+}
+
+extern "C" int64_t nb_gemm_prefill_f32_ws_bytes(int M, int N, int K) {
+    return f32_ws_bytes(M, N, K, PlanSpace::kLeast);
+}
+
+extern "C" int nb_gemm_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed,
+                                   const float* codebook, float* y, int64_t ldy, int M, int N,
+                                   int K, void* workspace, int64_t ws_bytes, void* stream) {
+    return prefill_f32("nb_gemm_prefill_f32", x, ldx, packed, codebook, y, ldy, M, N, K, workspace,
+                       ws_bytes, PlanSpace::kLeast, stream);
+}
+
+extern "C" int64_t nb_gemm_prefill_f32_best_ws_bytes(int M, int N, int K) {
+    return f32_ws_bytes(M, N, K, PlanSpace::kBest);
+}
+
+extern "C" int nb_gemm_prefill_f32_best(const float* x, int64_t ldx, const uint8_t* packed,
+                                        const float* codebook, float* y, int64_t ldy, int M, int N,
+                                        int K, void* workspace, int64_t ws_bytes, void* stream) {
+    return prefill_f32("nb_gemm_prefill_f32_best", x, ldx, packed, codebook, y, ldy, M, N, K,
+                       workspace, ws_bytes, PlanSpace::kBest, stream);
 }
 
 namespace {

@@ -142,24 +142,23 @@ int launch_dequant(const uint8_t* packed, const float* codebook, void* w,
 
 
 // Prefill GEMM with a packed weight (nb_prefill2.hip): the packed weight
-// dequantized into LDS tiles, bf16 MFMAs; arguments validated.  With a
-// workspace of at least prefill_split_bytes(M, N, K) bytes, a layer whose
+// dequantized into LDS tiles, bf16 MFMAs; arguments validated.  A layer whose
 // tile grid leaves CUs idle is split over K ranges (fp32 partial products in
-// the workspace, then one reduction launch); otherwise (workspace null) one
-// launch over all of K.
+// the workspace, then one reduction launch) where `space` allows it: kNone
+// one launch over all of K, no workspace; kLeast and kBest a workspace of
+// prefill_split_bytes(M, N, K, space) bytes, of which no more is touched.
+enum class PlanSpace { kNone, kLeast, kBest };
 int launch_prefill2(const void* x, int64_t ldx, const uint8_t* packed, const float* codebook,
                     void* y, int y_dtype, int64_t ldy, int M, int N, int K, void* workspace,
-                    int64_t ws_bytes, hipStream_t stream);
-int64_t prefill_split_bytes(int M, int N, int K);
-int64_t prefill_split_best_bytes(int M, int N, int K);
+                    PlanSpace space, hipStream_t stream);
+int64_t prefill_split_bytes(int M, int N, int K, PlanSpace space);
 // fp32 activations: x split into bf16 hi + lo in the workspace, then the
 // same kernel with three bf16 products per fp32 one (workspace of
-// prefill_f32_bytes(M, N, K) bytes, 256-byte aligned).
-int64_t prefill_f32_bytes(int M, int N, int K);
-int64_t prefill_f32_best_bytes(int M, int N, int K);
+// prefill_f32_bytes(M, N, K, space) bytes, 256-byte aligned; kLeast or kBest).
+int64_t prefill_f32_bytes(int M, int N, int K, PlanSpace space);
 int launch_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed, const float* codebook,
                        float* y, int64_t ldy, int M, int N, int K, void* workspace,
-                       int64_t ws_bytes, hipStream_t stream);
+                       PlanSpace space, hipStream_t stream);
 
 // Decode-step kernels (nb_decode.hip).
 int launch_add_rmsnorm(float* x, const float* y, const float* emb, const nb_decode_state* st,

@@ -515,11 +515,11 @@ float plan_time(const TileCost& c, int S, int M, int N, int K, int64_t cus, floa
 // 24.0 -> 11.7 / 13.3 us, 1024 x 4096 35 -> 12 us, 5000 x 1024 at M = 300 22 ->
 // 14.6 us, 2560 x 6912 at M = 700 55 -> 47 us; the sizes that the thresholds
 // were tuned on keep their plans or ones as fast.
-// A grid that reaches 0.6 of the CUs is split too where the caller's
-// workspace (ws_bytes, beyond what prefill_split_bytes asks for) holds the
-// partial products and the estimate is a tenth less: 2560 x 6912 at M = 1024 88
-// -> 56 us (three ranges of 256 x 128).
-PrefillPlan prefill_plan(int M, int N, int K, bool allow_split, int64_t ws_bytes) {
+// A grid that reaches 0.6 of the CUs is split too where the caller gave the
+// workspace of the fastest plan (kBest) and the estimate is a tenth less: 2560
+// x 6912 at M = 1024 88 -> 56 us (three ranges of 256 x 128).  The plan follows
+// from the shape and `space` alone, never from the size of the workspace.
+PrefillPlan prefill_plan(int M, int N, int K, PlanSpace space) {
     const int64_t cus = device_cu_count();
     const int nsteps = K / kBK;
     const int64_t limit = 4 * ((int64_t)N * K / 128 * 80);
@@ -533,7 +533,7 @@ PrefillPlan prefill_plan(int M, int N, int K, bool allow_split, int64_t ws_bytes
         }
     };
     for (const TileCost& c : kBf16Tiles) offer(c, 1);
-    if (!allow_split) return best;
+    if (space == PlanSpace::kNone) return best;
     int64_t full = 0;   // the grid of the largest tile that fills 0.6 of the CUs
     for (int i = 0; i < 3 && !full; ++i) {
         const int64_t g = grid_of(M, N, kBf16Tiles[i].BM, kBf16Tiles[i].BN);
@@ -550,7 +550,7 @@ PrefillPlan prefill_plan(int M, int N, int K, bool allow_split, int64_t ws_bytes
     } else {
         best_t *= 1.1f;   // (the estimates' error: split where it costs about the same)
     }
-    const int64_t most = full ? std::min(limit, ws_bytes) : limit;
+    const int64_t most = full && space != PlanSpace::kBest ? 0 : limit;
     for (const TileCost& c : kBf16Tiles) {
         for (int S = 2; S <= 8 && nsteps / S >= kMinSplitSteps; ++S) {
             if ((int64_t)S * M * N * 4 <= most) offer(c, S);
@@ -620,18 +620,15 @@ __global__ __launch_bounds__(256) void split_bf16_kernel(const float* __restrict
 
 inline int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
-}  // namespace
-
-int64_t prefill_split_bytes(int M, int N, int K) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
-    const PrefillPlan p = prefill_plan(M, N, K, true, 0);
+inline int64_t partial_bytes(const PrefillPlan& p, int M, int N) {
     return p.S > 1 ? (int64_t)p.S * M * N * 4 : 0;
 }
 
-int64_t prefill_split_best_bytes(int M, int N, int K) {
+}  // namespace
+
+int64_t prefill_split_bytes(int M, int N, int K, PlanSpace space) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
-    const PrefillPlan p = prefill_plan(M, N, K, true, INT64_MAX);
-    return std::max(p.S > 1 ? (int64_t)p.S * M * N * 4 : 0, prefill_split_bytes(M, N, K));
+    return partial_bytes(prefill_plan(M, N, K, space), M, N);
 }
 
 namespace {
@@ -672,34 +669,44 @@ int launch_tiles(Prefill2Args a, const PrefillPlan& p, void* workspace, hipStrea
 
 int launch_prefill2(const void* x, int64_t ldx, const uint8_t* packed, const float* codebook,
                     void* y, int y_dtype, int64_t ldy, int M, int N, int K, void* workspace,
-                    int64_t ws_bytes, hipStream_t stream) {
-    PrefillPlan p = prefill_plan(M, N, K, workspace != nullptr, ws_bytes);
-    if (p.S > 1 && ws_bytes < (int64_t)p.S * M * N * 4) p = prefill_plan(M, N, K, false, 0);
+                    PlanSpace space, hipStream_t stream) {
     return launch_tiles<false>({static_cast<const uint16_t*>(x), ldx, packed, codebook, y, ldy,
-                                y_dtype, M, N, K, 1, nullptr}, p, workspace, stream);
+                                y_dtype, M, N, K, 1, nullptr},
+                               prefill_plan(M, N, K, space), workspace, stream);
 }
 
-int64_t prefill_f32_bytes(int M, int N, int K) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
-    // (the size that callers may have stored: two bf16 parts of x, a codebook
-    // and the bf16 kernel's partial products; the codebook's part goes to
-    // partial products too)
+namespace {
+
+// The least workspace: two bf16 parts of x, a codebook's size and the bf16
+// kernel's partial products (the size that callers may have stored; what the
+// parts of x leave goes to partial products).
+int64_t prefill_f32_least(int M, int N, int K) {
     const int64_t xb = align256((int64_t)M * K * 2);
     const int64_t cb = align256((int64_t)N * (K / 128) * 8 * 4);
-    return 2 * xb + cb + prefill_split_bytes(M, N, K);
+    return 2 * xb + cb + prefill_split_bytes(M, N, K, PlanSpace::kLeast);
 }
 
-int64_t prefill_f32_best_bytes(int M, int N, int K) {
-    const int64_t least = prefill_f32_bytes(M, N, K);
-    if (least == 0) return 0;
-    const PrefillPlan p = prefill_f32_plan(M, N, K, 128LL << 20);
-    const int64_t part = p.S > 1 ? (int64_t)p.S * M * N * 4 : 0;
-    return std::max(least, align256((int64_t)M * K * 4) + part);
+// Partial products fit what the least workspace leaves beside the parts of x
+// (kLeast), or 128 MiB where that is more (kBest).
+PrefillPlan prefill_f32_plan(int M, int N, int K, PlanSpace space) {
+    const int64_t left = prefill_f32_least(M, N, K) - align256((int64_t)M * K * 4);
+    return prefill_f32_plan(M, N, K,
+                            space == PlanSpace::kBest ? std::max<int64_t>(left, 128LL << 20) : left);
+}
+
+}  // namespace
+
+int64_t prefill_f32_bytes(int M, int N, int K, PlanSpace space) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
+    const int64_t least = prefill_f32_least(M, N, K);
+    if (space != PlanSpace::kBest) return least;
+    return std::max(least, align256((int64_t)M * K * 4) +
+                               partial_bytes(prefill_f32_plan(M, N, K, space), M, N));
 }
 
 int launch_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed, const float* codebook,
                        float* y, int64_t ldy, int M, int N, int K, void* workspace,
-                       int64_t ws_bytes, hipStream_t stream) {
+                       PlanSpace space, hipStream_t stream) {
     GemvArgs rows;
     rows.x = x;
     rows.x_dtype = NB_F32;
@@ -733,8 +740,7 @@ int launch_prefill_f32(const float* x, int64_t ldx, const uint8_t* packed, const
     if (st) return st;
     return launch_tiles<true>({xs, 2 * (int64_t)K, packed, codebook, y, ldy, NB_F32, M, N, K, 1,
                                nullptr},
-                              prefill_f32_plan(M, N, K, ws_bytes - xbytes),
-                              w + xbytes, stream);
+                              prefill_f32_plan(M, N, K, space), w + xbytes, stream);
 }
 
 }  // namespace nb

@@ -380,7 +380,7 @@ def gemm_prefill(x: torch.Tensor, packed: torch.Tensor, codebook: torch.Tensor, 
     """y = x @ bf16(W).T for a 3-bit / 8-entry / block-128 packed W (N x K);
     x (M, K) bfloat16, row-contiguous, fp32 accumulation.
 
-    ``path``: "auto" (nb_gemm_prefill_split: the hand-written MFMA kernel,
+    ``path``: "auto" (nb_gemm_prefill_split_best: the hand-written MFMA kernel,
     the packed weight dequantized into LDS tiles; a layer whose tile grid
     would leave CUs idle -- few tokens, narrow layers -- is split over K
     ranges, with fp32 partial products in a workspace taken from torch's
@@ -408,7 +408,7 @@ def gemm_prefill(x: torch.Tensor, packed: torch.Tensor, codebook: torch.Tensor, 
     if path == "auto":
         nbytes = int(lib.nb_gemm_prefill_split_best_ws_bytes(M, N, K))
         ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
-        _lib.check(lib.nb_gemm_prefill_split(
+        _lib.check(lib.nb_gemm_prefill_split_best(
             x.data_ptr(), x.stride(0), packed.data_ptr(), codebook.data_ptr(), out.data_ptr(),
             _DT[out.dtype], out.stride(0), M, N, K, ws.data_ptr() if nbytes else None, nbytes,
             _stream(x)))
@@ -424,7 +424,7 @@ def gemm_prefill_f32(x: torch.Tensor, packed: torch.Tensor, codebook: torch.Tens
                      K: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """y = x @ W.T for fp32 x (M, K) against the exact fp32 codebook values of
     a 3-bit / 8-entry / block-128 packed W (N x K), y fp32 (M, N):
-    nb_gemm_prefill_f32, three bf16 products over the hi / lo parts of x and
+    nb_gemm_prefill_f32_best, three bf16 products over the hi / lo parts of x and
     W (each product to within 2^-16 of its size; few rows of a small layer:
     the exact fp32 products), the packed weight
     dequantized into LDS tiles, never materialised; a workspace from torch's
@@ -446,7 +446,7 @@ def gemm_prefill_f32(x: torch.Tensor, packed: torch.Tensor, codebook: torch.Tens
     lib = _lib.load()
     nbytes = int(lib.nb_gemm_prefill_f32_best_ws_bytes(M, N, K))
     ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
-    _lib.check(lib.nb_gemm_prefill_f32(
+    _lib.check(lib.nb_gemm_prefill_f32_best(
         x.data_ptr(), x.stride(0), packed.data_ptr(), codebook.data_ptr(), out.data_ptr(),
         out.stride(0), M, N, K, ws.data_ptr(), nbytes, _stream(x)))
     return out

@@ -632,3 +632,24 @@ def test_prefill_f32_validation(kw, status):
 
 def test_prefill_f32_empty_is_ok():
     assert prefill_f32(M=0) == _lib.NB_OK and prefill_f32(N=0) == _lib.NB_OK
+
+
+@pytest.mark.parametrize("name", ["nb_gemm_prefill_split", "nb_gemm_prefill_f32"])
+def test_prefill_best_entry_needs_its_own_workspace(name):
+    """The fastest plan is an entry point of its own: it refuses the least
+    workspace where its plan needs more, and the other one asks for no more
+    than before (0 where it does not split)."""
+    lib, f32 = _lib.load(), name.endswith("f32")
+    M, N, K = 1024, 2560, 6912
+    least = getattr(lib, name + "_ws_bytes")(M, N, K)
+    best = getattr(lib, name + "_best_ws_bytes")(M, N, K)
+    assert best > least and (f32 or least == 0)
+
+    def call(entry, ws, nbytes):
+        dtype = () if f32 else (_lib.NB_F32,)
+        return getattr(lib, entry)(FAKE, K, FAKE, FAKE, FAKE, *dtype, N, M, N, K, ws, nbytes, None)
+    assert call(name + "_best", FAKE, best - 1) == _lib.NB_EINVAL
+    assert _lib.last_error().startswith(f"{name}_best: workspace of {best - 1} bytes < {best}")
+    assert call(name + "_best", None, best) == _lib.NB_EINVAL
+    assert call(name + "_best", FAKE + 16, best) == _lib.NB_EALIGN
+    assert getattr(lib, name + "_best_ws_bytes")(M, N, 100) == 0

@@ -48,40 +48,72 @@ def test_f32_strided_rows(dev, pad):
     assert _case(dev, 20, 300, 256, pad).max() <= 1.0
 
 
+def _entry(f32, best):
+    """(the call, its workspace size) of an entry point; the call takes x,
+    packed, codebook, y, m, n, k, workspace and its size."""
+    lib, name = _lib.load(), "nb_gemm_prefill_f32" if f32 else "nb_gemm_prefill_split"
+    name += "_best" if best else ""
+    size, f = getattr(lib, name + "_ws_bytes"), getattr(lib, name)
+
+    def call(x, packed, cb, y, m, n, k, ws, nbytes):
+        dtype = () if f32 else (_lib.NB_F32,)
+        _lib.check(f(x.data_ptr(), k, packed.data_ptr(), cb.data_ptr(), y.data_ptr(), *dtype, n, m,
+                     n, k, ws.data_ptr() if ws is not None else None, nbytes,
+                     torch.cuda.current_stream().cuda_stream))
+    return call, size
+
+
+def _operands(dev, f32, m, n, k):
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    idx = torch.randint(0, 8, (n * k,), generator=g, device=dev, dtype=torch.uint8)
+    cb = torch.randn(n * k // 128, 8, generator=g, device=dev) * 0.02
+    x = torch.randn(m, k, generator=g, device=dev)
+    if not f32:
+        x, cb = x.bfloat16(), cb.bfloat16().float()
+    return idx, ops.pack(idx, 3), cb, x
+
+
 @pytest.mark.parametrize("f32", [True, False])
 @pytest.mark.parametrize("m,n,k", [
     (500, 7680, 2560), (290, 6912, 1280), (1000, 2560, 6912), (257, 2561, 4096), (40, 128, 384)])
 def test_plans_of_both_workspaces(dev, f32, m, n, k):
-    """The fastest plan (the workspace of *_best_ws_bytes) and the one of
-    *_ws_bytes write only their workspace and y.  fp32: the bound above; bf16:
+    """The fastest plan (the *_best entry points) and the one of the least
+    workspace write only their workspace and y.  fp32: the bound above; bf16:
     exact products of bf16 values in fp32 sums, (K / 32 + 40) 2^-24 sum |x w|."""
     print(f"[case] prefill plans {m}x{n}x{k} f32={f32}", flush=True)
-    lib = _lib.load()
-    g = torch.Generator(device=dev).manual_seed(m + n + k)
-    idx = torch.randint(0, 8, (n * k,), generator=g, device=dev, dtype=torch.uint8)
-    cb = torch.randn(n * k // 128, 8, generator=g, device=dev) * 0.02
-    packed = ops.pack(idx, 3)
-    x = torch.randn(m, k, generator=g, device=dev)
-    if not f32:
-        x, cb = x.bfloat16(), cb.bfloat16().float()
+    idx, packed, cb, x = _operands(dev, f32, m, n, k)
     w = cb.double().gather(1, idx.view(-1, 128).long()).view(n, k)
     ref, size = x.double() @ w.T, x.double().abs() @ w.T.abs()
     bound = (3 * 2.0 ** -18 + (3 * k / 32 + 48) * 2.0 ** -24 if f32 else (k / 32 + 40) * 2.0 ** -24) * size
-    name = "nb_gemm_prefill_f32" if f32 else "nb_gemm_prefill_split"
-    least = getattr(lib, name + "_ws_bytes")(m, n, k)
-    best = getattr(lib, name + "_best_ws_bytes")(m, n, k)
-    assert best >= least
-    for nbytes in {least, best}:
+    assert _entry(f32, True)[1](m, n, k) >= _entry(f32, False)[1](m, n, k)
+    for best in (False, True):
+        call, ws_bytes = _entry(f32, best)
+        nbytes = ws_bytes(m, n, k)
         ws = torch.full((nbytes + 4096,), 0xff, dtype=torch.uint8, device=dev)
         y = torch.empty(m + 1, n, device=dev)
         y[m] = 7.0
-        args = (m, n, k, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
-        if f32:
-            st = lib.nb_gemm_prefill_f32(x.data_ptr(), k, packed.data_ptr(), cb.data_ptr(),
-                                         y.data_ptr(), n, *args)
-        else:
-            st = lib.nb_gemm_prefill_split(x.data_ptr(), k, packed.data_ptr(), cb.data_ptr(),
-                                           y.data_ptr(), _lib.NB_F32, n, *args)
-        _lib.check(st)
+        call(x, packed, cb, y, m, n, k, ws, nbytes)
         assert (ws[nbytes:] == 0xff).all() and (y[m] == 7.0).all()
         assert ((y[:m].double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("f32", [True, False])
+@pytest.mark.parametrize("m,n,k", [(1024, 2560, 6912), (500, 7680, 2560), (867, 8716, 3840),
+                                   (64, 2560, 2560)])
+def test_a_larger_workspace_changes_nothing(dev, f32, m, n, k):
+    """Bytes past *_ws_bytes are not touched -- none at all where that is 0,
+    so that calls on several streams may share them -- and the result's bits
+    do not depend on the workspace's size."""
+    print(f"[case] prefill workspace {m}x{n}x{k} f32={f32}", flush=True)
+    _, packed, cb, x = _operands(dev, f32, m, n, k)
+    most = _entry(f32, True)[1](m, n, k)
+    for best in (False, True):
+        call, ws_bytes = _entry(f32, best)
+        need = ws_bytes(m, n, k)
+        ys = []
+        for nbytes in (need, need + 512, most + (160 << 20)):
+            ws = torch.full((nbytes,), 0xff, dtype=torch.uint8, device=dev) if nbytes else None
+            ys.append(torch.empty(m, n, device=dev))
+            call(x, packed, cb, ys[-1], m, n, k, ws, nbytes)
+            assert ws is None or (ws[need:] == 0xff).all()
+        assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
