@@ -39,7 +39,7 @@
 // one chain a wave 2-3e-7.
 //
 // Formats: 2/3/4-bit with 2^bits entries, BS 64/128/256, K % 128 == 0 and
-// K % BS == 0.
+// K % BS == 0, up to 16 rows; up to 64 for 3-bit / BS 128.
 #include "nb_device.h"
 #include "nb_internal.h"
 #include "nb_lookup.h"
@@ -211,8 +211,9 @@ __global__ __launch_bounds__(64 * max_waves(TM)) void gemm_rows_f32_kernel(RowsA
     }
 }
 
-// Waves a workgroup: about six a CU over the grid, each with the same number
-// of units, at most five.  (More waves add their start and the final sum,
+// Waves a workgroup: about six a CU over the grid, with equal numbers of units
+// to within one, at most five a wave unless the workgroup's wave limit forces
+// more (2560 x 16384: eight).  (More waves add their start and the final sum,
 // fewer leave SIMDs idle: 2560 x 2560 at M = 8 in 8.6 us at six a CU, 10.0
 // at 12, 8.2 at four; 6912 x 2560 in 12.8 / 13.1 / 14.3 us; 2560 x 6912 with
 // six units a wave 16.6 us, with four 15.8.)
@@ -235,14 +236,21 @@ void launch_rows(const RowsArgs& a, hipStream_t stream) {
                        dim3(64 * waves), std::max(tables, red), stream, a);
 }
 
+// More than one activation tile only for the format that nb_gemm_prefill_f32
+// takes (nb_gemv stops at 16 rows).
+constexpr bool many_rows(int bits, int block_size) { return bits == 3 && block_size == 128; }
+
 template <int BITS, int BS>
 void launch_rows_m(const RowsArgs& a, hipStream_t stream) {
-    switch ((a.M + 15) / 16) {
-        case 1: launch_rows<BITS, BS, 1>(a, stream); break;
-        case 2: launch_rows<BITS, BS, 2>(a, stream); break;
-        case 3: launch_rows<BITS, BS, 3>(a, stream); break;
-        default: launch_rows<BITS, BS, 4>(a, stream); break;
+    if constexpr (many_rows(BITS, BS)) {
+        switch ((a.M + 15) / 16) {
+            case 1: break;
+            case 2: return launch_rows<BITS, BS, 2>(a, stream);
+            case 3: return launch_rows<BITS, BS, 3>(a, stream);
+            default: return launch_rows<BITS, BS, 4>(a, stream);
+        }
     }
+    launch_rows<BITS, BS, 1>(a, stream);
 }
 
 template <int BITS>
@@ -257,9 +265,10 @@ void launch_rows_bs(const RowsArgs& a, int block_size, hipStream_t stream) {
 }  // namespace
 
 bool gemm_rows_f32_eligible(const GemvArgs& a) {
-    if (a.x_dtype != NB_F32 || a.M < 1 || a.M > 16 * kMaxTiles) return false;
+    if (a.x_dtype != NB_F32 || a.M < 1) return false;
     if (a.bits < 2 || a.bits > 4 || a.n_entries != (1 << a.bits)) return false;
     if (a.block_size != 64 && a.block_size != 128 && a.block_size != 256) return false;
+    if (a.M > (many_rows(a.bits, a.block_size) ? 16 * kMaxTiles : 16)) return false;
     if (a.K <= 0 || a.K % kUnitK != 0 || a.K % a.block_size != 0) return false;
     // dword loads of the stream, 16-byte loads of the codebook and x
     if (reinterpret_cast<uintptr_t>(a.packed) % 4 != 0) return false;

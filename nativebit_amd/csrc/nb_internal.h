@@ -123,8 +123,9 @@ int launch_gemv(const GemvArgs& a, hipStream_t stream);
 // The bf16-activation MFMA GEMV; returns 1 (launching nothing) when the
 // problem is outside its 3-bit / 8-entry / block-128 / aligned domain.
 int launch_gemv_mfma(const GemvArgs& a, hipStream_t stream);
-// fp32 activations of up to 64 rows, exact fp32 products on fp32 MFMAs
-// (nb_gemm_rows.hip): whether it takes the operands, and its launch.
+// fp32 activations of up to 16 rows (3-bit / block-128: 64), exact fp32
+// products on fp32 MFMAs (nb_gemm_rows.hip): whether it takes the operands,
+// and its launch.
 bool gemm_rows_f32_eligible(const GemvArgs& a);
 int launch_gemm_rows_f32(const GemvArgs& a, hipStream_t stream);
 int launch_unpack(const uint8_t* packed, uint8_t* out, int64_t count, int bits,

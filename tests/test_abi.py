@@ -594,6 +594,16 @@ def test_rmsnorm_rows_vocab_ignored_without_lookup():
                                        256, 1e-6, None) == _lib.NB_OK
 
 
+def test_row_kernels_that_no_call_reaches_are_not_built():
+    """nb_gemv takes 16 rows of fp32 x, nb_gemm_prefill_f32 up to 64 on the
+    row kernel, in the 3-bit / block-128 format only: one 16-row tile for
+    every format, two to four for that one."""
+    out = subprocess.run(["nm", "-C", _lib.LIB_PATH], capture_output=True, text=True, check=True).stdout
+    built = set(re.findall(r"gemm_rows_f32_kernel<(\d+), (\d+), (\d+)>", out))
+    want = {(b, s, "1") for b in "234" for s in ("64", "128", "256")}
+    assert built == want | {("3", "128", t) for t in "234"}
+
+
 def test_prefill_f32_ws_bytes():
     lib = _lib.load()
     # bf16 hi and lo parts of x (256-byte rounded), the residual codebook,
