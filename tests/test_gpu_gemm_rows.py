@@ -1,11 +1,12 @@
-"""The fp32 multi-row kernel of nb_gemv (nb_gemm_rows.hip): exact codebook
-values, fp32 activations, at the edges of its 16-row tiles, 128-column units
-and wave splits, against fp64.
+"""The fp32 multi-row kernel of nb_gemv and nb_gemm_prefill_f32
+(nb_gemm_rows.hip): exact codebook values, fp32 activations, at the edges of
+its 16-row tiles, 128-column units and wave splits, against fp64.
 
-Bound: a product passes at most 8 roundings in its accumulator, 4 in the
-unit's tree, one per unit of the wave's sum and one of the workgroup's (formed
-in fp64), so |error| <= n 2^-24 sum |x w| with n = 13 + K / 128 (first order;
-1 % is added for the higher ones)."""
+Bound: a product passes at most 8 roundings in its accumulator (32 over 16
+rows), 4 in the unit's tree, one per unit of the wave's sum and one of the
+workgroup's (formed in fp64), so |error| <= n 2^-24 sum |x w| with n = 13 + K /
+128 (37 + K / 128 over 16 rows; first order; 1 % is added for the higher
+ones)."""
 import numpy as np
 import pytest
 import torch
@@ -24,16 +25,17 @@ def _layer(n, k, bits, bs, seed):
     return O.pack(idx, bits), cb, O.dequant(idx, cb, bs, n * k).reshape(n, k)
 
 
-def _check(y, x, w, k, slack=0.0):
+def _check(y, x, w, k, slack=0.0, roundings=13):
     x, w = x.astype(np.float64), w.astype(np.float64)
     ref, mag = x @ w.T, np.abs(x) @ np.abs(w).T
-    bound = 1.01 * (13 + k / 128) * 2.0 ** -24 * mag + slack * np.abs(ref)
+    bound = 1.01 * (roundings + k / 128) * 2.0 ** -24 * mag + slack * np.abs(ref)
     assert np.all(np.abs(y - ref) <= bound), float((np.abs(y - ref) / bound).max())
 
 
 @pytest.mark.parametrize("bits,bs", [(2, 64), (2, 256), (3, 64), (3, 128), (4, 128), (4, 256)])
 @pytest.mark.parametrize("n,k,m", [(1, 256, 2), (15, 256, 16), (17, 768, 15), (130, 2560, 3),
-                                   (513, 1280, 9), (64, 8448, 2), (4097, 256, 5)])
+                                   (513, 1280, 9), (64, 8448, 2), (4097, 256, 5),
+                                   (64, 2048, 16)])   # the last: 16 waves of one unit
 def test_rows_vs_f64(dev, bits, bs, n, k, m):
     print(f"[case] rows bits={bits} bs={bs} {n}x{k} m={m}", flush=True)
     packed, cb, w = _layer(n, k, bits, bs, n + k + m)
@@ -41,6 +43,22 @@ def test_rows_vs_f64(dev, bits, bs, n, k, m):
     y = ops.gemv(torch.from_numpy(x).to(dev), torch.from_numpy(packed).to(dev),
                  torch.from_numpy(cb).to(dev), n, k, bits=bits, block_size=bs)
     _check(y.cpu().numpy(), x, w, k)
+
+
+# 2..4 activation tiles (nb_gemm_prefill_f32 up to 4e8 products, 3-bit / BS
+# 128): full and ragged ones; two units a wave, one or two, 6-7 and 12-13
+@pytest.mark.parametrize("m", [17, 31, 32, 33, 48, 49, 63, 64])
+@pytest.mark.parametrize("n,k", [(2561, 2304), (2561, 1408), (15, 6272), (300, 12928), (40, 128)])
+def test_rows_of_several_tiles_vs_f64(dev, n, k, m):
+    """The exact products: a bound of fp32 roundings alone, far below the
+    2^-16 of the three bf16 products that larger sizes run on."""
+    print(f"[case] rows tiles {n}x{k} m={m}", flush=True)
+    assert m * n * k <= 400_000_000
+    packed, cb, w = _layer(n, k, 3, 128, n + k + m)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    y = ops.gemm_prefill_f32(torch.from_numpy(x).to(dev), torch.from_numpy(packed).to(dev),
+                             torch.from_numpy(cb).to(dev), n, k)
+    _check(y.cpu().numpy(), x, w, k, roundings=37)
 
 
 def test_rows_one_row_odd_units_and_forms(dev):

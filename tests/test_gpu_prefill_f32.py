@@ -1,6 +1,6 @@
 """nb_gemm_prefill_f32 in one kernel (x and W as bf16 hi + lo parts, three
-products a step) and its few-rows route, at edges of tiles, blocks and K
-ranges, against fp64.
+products a step) at edges of tiles, blocks and K ranges, against fp64, and
+the way to its few-rows route (whose kernel has tests and a bound of its own).
 
 Bound: hi + lo is x, and W, to 2^-18, and lo.lo (at most 2^-18 |x w|) is
 dropped: 3 * 2^-18 sum |x w|; the fp32 sums run over 3 K / 32 MFMAs, their
