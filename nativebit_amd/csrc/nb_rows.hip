@@ -190,16 +190,54 @@ __global__ __launch_bounds__(256) void silu_mul_rows_kernel(const float* __restr
 }
 
 // ---------------------------------------------------------------------------
-// RoPE + cache append: a workgroup takes kRT tokens of one head of one
-// sequence.  The rows are read and q and v written a wave per token, lanes
-// along the head's pairs; the rotated keys pass through LDS so that they are
-// written along positions, the transposed cache's fast index (written by the
-// threads that rotate them, every 4-byte store had a cache line of its own:
-// 15.5 us for 500 tokens of 20 heads of 128, 31 MB; now 9.8).
+// RoPE + cache append, two forms with the same arithmetic (launch_rope_kv_rows
+// chooses).
+//
+// Few elements: a wave per token and head, lanes along the head's pairs; the
+// rotated keys are written by the lanes that form them, each 4-byte store to
+// a cache line of its own in the transposed cache.  Latency bound: 2.2-2.5 us
+// for one token (any head count up to 160), 2.7 for 33 of 6 heads of 128,
+// where the form below takes 2.8-3.3 and 4.9.
+//
+// Many: a workgroup takes kRT tokens of one head of one sequence.  The rows
+// are read and q and v written a wave per token; the rotated keys pass
+// through LDS so that they are written along positions, the transposed
+// cache's fast index: 512 tokens of 20 heads of 128 (31 MB) in 8.1 us against
+// 15.5 in the form above.
 // ---------------------------------------------------------------------------
 constexpr int kRT = 32;
 constexpr int kRopeThreads = 256;
 constexpr int kRopeMaxD = 128;
+
+// x * cos2 + rotate(x) * sin2 of one pair (generate_torch.py:54-59)
+__device__ __forceinline__ float2 rope_pair(float a, float b, float c, float s) {
+    return make_float2(__fadd_rn(__fmul_rn(a, c), __fmul_rn(-b, s)),
+                       __fadd_rn(__fmul_rn(b, c), __fmul_rn(a, s)));
+}
+
+__global__ __launch_bounds__(64) void rope_kv_token_kernel(
+    const float* __restrict__ qkv, float* __restrict__ k_cache, float* __restrict__ v_cache,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t, int pos0,
+    float* __restrict__ q_out, int D, int ctx) {
+    const int t = blockIdx.x, hd = blockIdx.y, b = blockIdx.z, n_head = gridDim.y;
+    const int C = n_head * D, half = D / 2, pos = pos0 + t;
+    const float scale = 1.0f / sqrtf((float)D);
+    const int64_t tok = (int64_t)b * gridDim.x + t, bh = (int64_t)b * n_head + hd;
+    const float* row = qkv + tok * 3 * C + hd * D;
+    float* qo = q_out + tok * C + hd * D;
+    float* ko = k_cache + bh * D * ctx + pos;
+    float* vo = v_cache + (bh * ctx + pos) * D;
+    for (int i = threadIdx.x; i < half; i += 64) {
+        const float c = cos_t[(int64_t)pos * half + i], s = sin_t[(int64_t)pos * half + i];
+        const float2 q = rope_pair(row[2 * i], row[2 * i + 1], c, s);
+        const float2 k = rope_pair(row[C + 2 * i], row[C + 2 * i + 1], c, s);
+        qo[2 * i] = __fmul_rn(q.x, scale);
+        qo[2 * i + 1] = __fmul_rn(q.y, scale);
+        ko[(int64_t)(2 * i) * ctx] = k.x;
+        ko[(int64_t)(2 * i + 1) * ctx] = k.y;
+    }
+    for (int d = threadIdx.x; d < D; d += 64) vo[d] = row[2 * C + d];
+}
 
 __global__ __launch_bounds__(kRopeThreads) void rope_kv_rows_kernel(
     const float* __restrict__ qkv, float* __restrict__ k_cache, float* __restrict__ v_cache,
@@ -221,14 +259,13 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kv_rows_kernel(
         float* vo = v_cache + ((int64_t)bh * ctx + pos) * D;
         for (int i = lane; i < half; i += 64) {
             const float c = cos_t[(int64_t)pos * half + i], s = sin_t[(int64_t)pos * half + i];
-            const float q0 = row[2 * i], q1 = row[2 * i + 1];
-            const float k0 = row[C + 2 * i], k1 = row[C + 2 * i + 1];
+            const float2 q = rope_pair(row[2 * i], row[2 * i + 1], c, s);
+            const float2 k = rope_pair(row[C + 2 * i], row[C + 2 * i + 1], c, s);
             const float v0 = row[2 * C + 2 * i], v1 = row[2 * C + 2 * i + 1];
-            // x * cos2 + rotate(x) * sin2 (generate_torch.py:54-59), q then * scale
-            qo[2 * i] = __fmul_rn(__fadd_rn(__fmul_rn(q0, c), __fmul_rn(-q1, s)), scale);
-            qo[2 * i + 1] = __fmul_rn(__fadd_rn(__fmul_rn(q1, c), __fmul_rn(q0, s)), scale);
-            ks[2 * i][t] = __fadd_rn(__fmul_rn(k0, c), __fmul_rn(-k1, s));
-            ks[2 * i + 1][t] = __fadd_rn(__fmul_rn(k1, c), __fmul_rn(k0, s));
+            qo[2 * i] = __fmul_rn(q.x, scale);
+            qo[2 * i + 1] = __fmul_rn(q.y, scale);
+            ks[2 * i][t] = k.x;
+            ks[2 * i + 1][t] = k.y;
             vo[2 * i] = v0;
             vo[2 * i + 1] = v1;
         }
@@ -393,6 +430,19 @@ int launch_rope_kv_rows(const float* qkv, float* k_cache, float* v_cache, const 
                         const float* sin_t, int pos0, int T, float* q_out, int batch, int n_head,
                         int D, int ctx, hipStream_t stream) {
     static_assert(kRopeMaxD >= kRowsMaxD, "the callers' largest head dim");
+    // One token, or up to 200 000 elements: with more the scattered stores
+    // cost more than the pass through LDS.  Both are as fast at 1900 tokens
+    // times heads of D = 128, 3900 of 64, 5900 of 32 and 9500 of 16 (4 to 60
+    // heads); with 160 heads of 128 already between 4 tokens (3.3 us against
+    // 3.5) and 8 (4.8 against 3.8).
+    constexpr int kMaxYZ = 65535;   // of a grid
+    const int64_t heads = (int64_t)batch * n_head;
+    if (batch <= kMaxYZ && n_head <= kMaxYZ &&
+        (T == 1 || (heads * T * D <= 200000 && (T <= 4 || heads < 128)))) {
+        hipLaunchKernelGGL(rope_kv_token_kernel, dim3(T, n_head, batch), dim3(64), 0, stream, qkv,
+                           k_cache, v_cache, cos_t, sin_t, pos0, q_out, D, ctx);
+        return check_launch("nb_rope_kv_rows");
+    }
     const int tiles = (T + kRT - 1) / kRT;
     hipLaunchKernelGGL(rope_kv_rows_kernel, dim3((unsigned)(batch * n_head * tiles)),
                        dim3(kRopeThreads), 0, stream, qkv, k_cache, v_cache, cos_t, sin_t, pos0, T,

@@ -22,7 +22,9 @@ def stream():
 
 @pytest.mark.parametrize("B,H,D,ctx,pos0,T", [
     (3, 5, 128, 96, 40, 1), (2, 3, 128, 132, 0, 33), (3, 2, 64, 100, 31, 64), (2, 3, 32, 72, 7, 31),
-    (2, 2, 128, 40, 0, 20), (2, 2, 6, 70, 1, 65)])
+    (2, 2, 128, 40, 0, 20), (2, 2, 6, 70, 1, 65),
+    # the batch through LDS, a sequence a wave per token and head; one token of many heads
+    (3, 5, 128, 132, 3, 120), (2, 3, 64, 840, 0, 800), (40, 64, 128, 8, 5, 1)])
 def test_batch_equals_sequences(dev, B, H, D, ctx, pos0, T):
     print(f"[case] rows batch B={B} H={H} D={D} ctx={ctx} pos0={pos0} T={T}", flush=True)
     lib, C = _lib.load(), H * D
