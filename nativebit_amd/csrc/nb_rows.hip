@@ -279,8 +279,8 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kv_rows_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// causal attention of T queries: grid (n_head, ceil(T / kQB)), 256 threads.
-// The workgroup holds kQB queries of one head and walks the keys in tiles
+// causal attention of T queries: grid (batch * n_head, ceil(T / kQB)), 256
+// threads.  The workgroup holds kQB queries of one head and walks the keys in tiles
 // of kKT positions through LDS with an online softmax (running max and sum
 // per query); query t sees positions 0 .. pos0 + t.  Head dims past D (up
 // to a multiple of 4) are zero in LDS, so the dot products run over float4
@@ -302,14 +302,16 @@ __global__ __launch_bounds__(kAttThreads) void attention_rows_kernel(
     __shared__ __align__(16) float ks[kRowsMaxD][kKPitch];   // keys transposed: [dim][position]
     __shared__ __align__(16) float vs[kKT][kQPitch];
     __shared__ __align__(16) float ps[kQB][kKPitch];
-    const int hd = blockIdx.x, t0 = blockIdx.y * kQB;
+    const int bh = blockIdx.x, t0 = blockIdx.y * kQB;
+    const int b = bh / n_head, hd = bh - b * n_head;
     const int tid = threadIdx.x;
     const int C = n_head * D;
+    const int64_t row0 = (int64_t)b * T;   // of q and out
     const int D4 = (D + 3) & ~3;
     const int nq = min(kQB, T - t0);
     for (int e = tid; e < kQB * kQPitch; e += kAttThreads) {
         const int i = e / kQPitch, d = e - i * kQPitch;
-        qs[i][d] = i < nq && d < D ? q[(int64_t)(t0 + i) * C + hd * D + d] : 0.f;
+        qs[i][d] = i < nq && d < D ? q[(row0 + t0 + i) * C + hd * D + d] : 0.f;
     }
     typedef __attribute__((ext_vector_type(2))) float f2;
     // scores: thread (sq, sp) takes query sq and keys 2 sp, 2 sp + 1
@@ -319,8 +321,8 @@ __global__ __launch_bounds__(kAttThreads) void attention_rows_kernel(
     f4 o0 = {0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;  // per query, kept by its 32 threads alike
     const int last = pos0 + t0 + nq - 1;  // the last position any query sees
-    const float* kt = k_cache + (int64_t)hd * D * ctx;
-    const float* vc = v_cache + (int64_t)hd * ctx * D;
+    const float* kt = k_cache + (int64_t)bh * D * ctx;
+    const float* vc = v_cache + (int64_t)bh * ctx * D;
     for (int p0 = 0; p0 <= last; p0 += kKT) {
         const int np = min(kKT, last + 1 - p0);
         __syncthreads();  // the previous tile is no longer read
@@ -392,7 +394,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_rows_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int d = 4 * og + j;
-            if (d < D) store_out(out, out_dtype, (int64_t)(t0 + oq) * C + hd * D + d, o0[j] / l_run);
+            if (d < D) store_out(out, out_dtype, (row0 + t0 + oq) * C + hd * D + d, o0[j] / l_run);
         }
     }
 }
@@ -460,13 +462,9 @@ int launch_attention_rows(const float* q, const float* k_cache, const float* v_c
         return launch_attention_mfma(q, k_cache, v_cache, pos0, T, out, out_dtype, batch, n_head, D,
                                      ctx, stream);
     }
-    for (int b = 0; b < batch; ++b) {
-        const int64_t rows = (int64_t)b * T * n_head * D, cache = (int64_t)b * n_head * D * ctx;
-        void* o = static_cast<char*>(out) + rows * (out_dtype == NB_BF16 ? 2 : 4);
-        hipLaunchKernelGGL(attention_rows_kernel, dim3(n_head, (T + kQB - 1) / kQB),
-                           dim3(kAttThreads), 0, stream, q + rows, k_cache + cache, v_cache + cache,
-                           pos0, T, o, out_dtype, n_head, D, ctx);
-    }
+    hipLaunchKernelGGL(attention_rows_kernel, dim3(batch * n_head, (T + kQB - 1) / kQB),
+                       dim3(kAttThreads), 0, stream, q, k_cache, v_cache, pos0, T, out, out_dtype,
+                       n_head, D, ctx);
     return check_launch("nb_attention_rows");
 }
 

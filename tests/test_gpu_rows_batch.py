@@ -24,7 +24,7 @@ def stream():
     (3, 5, 128, 96, 40, 1), (2, 3, 128, 132, 0, 33), (3, 2, 64, 100, 31, 64), (2, 3, 32, 72, 7, 31),
     (2, 2, 128, 40, 0, 20), (2, 2, 6, 70, 1, 65),
     # the batch through LDS, a sequence a wave per token and head; one token of many heads
-    (3, 5, 128, 132, 3, 120), (2, 3, 64, 840, 0, 800), (40, 64, 128, 8, 5, 1)])
+    (3, 5, 128, 132, 3, 120), (2, 3, 64, 840, 0, 800), (40, 64, 64, 8, 5, 1)])
 def test_batch_equals_sequences(dev, B, H, D, ctx, pos0, T):
     print(f"[case] rows batch B={B} H={H} D={D} ctx={ctx} pos0={pos0} T={T}", flush=True)
     lib, C = _lib.load(), H * D
@@ -62,6 +62,29 @@ def test_batch_equals_sequences(dev, B, H, D, ctx, pos0, T):
     rot = torch.stack((kk[:, :, :, 0] * c - kk[:, :, :, 1] * s,
                        kk[:, :, :, 1] * c + kk[:, :, :, 0] * s), 3).reshape(B, H, D, T)
     assert (k[..., span] - rot).abs().max() <= 4 * 2.0 ** -24 * kk.abs().max()
+
+
+@pytest.mark.parametrize("D,ctx,pos0", [(32, 40, 20), (128, 40, 20), (128, 40, 36), (128, 41, 20)])
+def test_a_batch_is_one_launch(dev, D, ctx, pos0):
+    """nb_rope_kv_batch and nb_attention_batch are one graph node each, on
+    every kernel that they choose from (heads of 32, few positions, the MFMA
+    kernel, rows of keys without 16-byte alignment)."""
+    lib, B, H = _lib.load(), 5, 2
+    qkv = torch.randn(B, 1, 3 * H * D, device=dev)
+    k, v = torch.zeros(B, H, D, ctx, device=dev), torch.zeros(B, H, ctx, D, device=dev)
+    q, out = torch.empty(B, 1, H * D, device=dev), torch.empty(B, 1, H * D, device=dev)
+    cos, sin = (t.to(dev).contiguous() for t in precompute_rope(D, ctx))
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        _lib.check(lib.nb_rope_kv_batch(P(qkv), P(k), P(v), P(cos), P(sin), pos0, 1, P(q), B, H, D,
+                                        ctx, stream()))
+        _lib.check(lib.nb_attention_batch(P(q), P(k), P(v), pos0, 1, P(out), _lib.NB_F32, B, H, D,
+                                          ctx, stream()))
+    nodes = ctypes.c_size_t(0)
+    get_nodes = lib.hipGraphGetNodes   # (of the HIP runtime that the library is linked to)
+    get_nodes.restype, get_nodes.argtypes = ctypes.c_int, [ctypes.c_void_p] * 3
+    assert get_nodes(graph.raw_cuda_graph(), None, ctypes.byref(nodes)) == 0
+    assert nodes.value == 2
 
 
 @pytest.mark.parametrize("n", [1, 5, 1024, 4097])
