@@ -456,9 +456,14 @@ int launch_attention_rows(const float* q, const float* k_cache, const float* v_c
                           int T, void* out, int out_dtype, int batch, int n_head, int D, int ctx,
                           hipStream_t stream) {
     // fp32 MFMAs where the layout allows 16-byte loads; up to 32 positions at
-    // head dim 128 the vector kernel below is as fast or faster (16 queries
-    // from position 0: 8.0 us against 8.9; 64: 9.3 against 9.0)
-    if (attention_mfma_eligible(q, k_cache, v_cache, D, ctx) && (D < 128 || pos0 + T > 32)) {
+    // head dim 128 the vector kernel below is as fast or faster while its
+    // workgroups leave CUs idle (16 queries from position 0, 20 heads 8.1 us
+    // against 8.8, 60 heads 8.3 against 8.9), from 128 heads over the batch on
+    // it is not (160 heads 10.1 against 9.2, 320 heads 16.7 against 10.3; one
+    // query 7.8 against 7.9 and 9.2 against 8.4).  Over 32 positions, 20
+    // heads: 16 queries up to position 48 8.8 against 8.8, 64 9.2 against 8.9.
+    if (attention_mfma_eligible(q, k_cache, v_cache, D, ctx) &&
+        (D < 128 || pos0 + T > 32 || (int64_t)batch * n_head >= 128)) {
         return launch_attention_mfma(q, k_cache, v_cache, pos0, T, out, out_dtype, batch, n_head, D,
                                      ctx, stream);
     }

@@ -49,6 +49,7 @@ def inputs(H, D, ctx, T, seed):
 @pytest.mark.parametrize("H,ctx,pos0,T", [
     (2, 64, 0, 64), (3, 68, 0, 65), (1, 128, 63, 1), (1, 128, 64, 1), (2, 260, 47, 17),
     (25, 132, 100, 16), (49, 80, 48, 31), (2, 1024, 1007, 17), (1, 320, 255, 33), (2, 300, 0, 300),
+    (130, 32, 3, 9),
     (2, 66, 40, 20)])   # the last: rows of keys without 16-byte alignment
 def test_tile_edges(dev, D, H, ctx, pos0, T):
     print(f"[case] attention mfma D={D} H={H} ctx={ctx} pos0={pos0} T={T}", flush=True)
