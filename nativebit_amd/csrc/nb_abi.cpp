@@ -766,11 +766,11 @@ int check_rows_attention(const char* fn, int pos0, int T, int n_head, int head_d
 }  // namespace
 
 namespace {
-// Sequences of a batched row call; rows * heads stay in a grid's range.
-int check_batch_size(const char* fn, int batch, int T, int n_head) {
+// Sequences of a batched row call (the kernels count its heads in an int).
+int check_batch_size(const char* fn, int batch, int n_head) {
     if (batch < 0) return fail(NB_EINVAL, "%s: batch=%d < 0", fn, batch);
-    if ((int64_t)batch * n_head * (T / 16 + 1) >= (1LL << 30)) {
-        return fail(NB_EUNSUPPORTED, "%s: batch=%d n_head=%d T=%d too large", fn, batch, n_head, T);
+    if ((int64_t)batch * n_head >= (1LL << 31)) {
+        return fail(NB_EUNSUPPORTED, "%s: batch=%d n_head=%d too large", fn, batch, n_head);
     }
     return NB_OK;
 }
@@ -780,7 +780,7 @@ int rope_kv(const char* fn, const float* qkv, float* k_cache, float* v_cache, co
             int ctx, void* stream) {
     int st = check_rows_attention(fn, pos0, T, n_head, head_dim, ctx);
     if (st) return st;
-    st = check_batch_size(fn, batch, T, n_head);
+    st = check_batch_size(fn, batch, n_head);
     if (st || batch == 0) return st;
     if (!qkv || !k_cache || !v_cache || !cos_t || !sin_t || !q_out) {
         return fail(NB_EINVAL, "%s: NULL pointer", fn);
@@ -801,7 +801,7 @@ int attention(const char* fn, const float* q, const float* k_cache, const float*
               void* stream) {
     int st = check_rows_attention(fn, pos0, T, n_head, head_dim, ctx);
     if (st) return st;
-    st = check_batch_size(fn, batch, T, n_head);
+    st = check_batch_size(fn, batch, n_head);
     if (st || batch == 0) return st;
     if (out_dtype != NB_F32 && out_dtype != NB_BF16) return fail(NB_EINVAL, "%s: out_dtype=%d", fn, out_dtype);
     if (!q || !k_cache || !v_cache || !out) return fail(NB_EINVAL, "%s: NULL pointer", fn);

@@ -65,7 +65,7 @@ struct AttArgs {
     void* out;              // [batch][T][n_head * D]
     int out_dtype;
     int pos0, T, n_head, ctx;
-    int heads;              // batch * n_head
+    int head0, heads;       // heads of this launch, of the batch * n_head
     int qtiles;             // query tiles of a head
 };
 
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attention_mfma_kernel(AttArgs 
     const int per_group = kHeads * a.qtiles;
     const int group = blockIdx.x / per_group, i0 = blockIdx.x - group * per_group;
     const int in_group = min(kHeads, a.heads - group * kHeads);
-    const int bh = group * kHeads + i0 % in_group;
+    const int bh = a.head0 + group * kHeads + i0 % in_group;
     const int qt0 = a.qtiles - 1 - i0 / in_group;
     const int t0 = qt0 * 16;
     const int C = a.n_head * D;
@@ -319,11 +319,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attention_mfma_kernel(AttArgs 
 }
 
 template <int D>
-void launch_att(AttArgs a, hipStream_t stream) {
+void launch_att(AttArgs a, int64_t heads, hipStream_t stream) {
     a.qtiles = (a.T + 15) / 16;
     const size_t lds = (size_t)kWaves * 16 * (D + 4 + 2) * 4;
-    hipLaunchKernelGGL((attention_mfma_kernel<D>), dim3(a.heads * a.qtiles), dim3(64 * kWaves),
-                       lds, stream, a);
+    for_head_ranges(heads, a.qtiles, 64 * kWaves, [&](int head0, int count) {
+        a.head0 = head0;
+        a.heads = count;
+        hipLaunchKernelGGL((attention_mfma_kernel<D>), dim3((unsigned)count * a.qtiles),
+                           dim3(64 * kWaves), lds, stream, a);
+    });
 }
 
 }  // namespace
@@ -338,11 +342,11 @@ bool attention_mfma_eligible(const float* q, const float* k, const float* v, int
 int launch_attention_mfma(const float* q, const float* k, const float* v, int pos0, int T,
                           void* out, int out_dtype, int batch, int n_head, int D, int ctx,
                           hipStream_t stream) {
-    AttArgs a = {q, k, v, out, out_dtype, pos0, T, n_head, ctx, batch * n_head, 0};
+    const AttArgs a = {q, k, v, out, out_dtype, pos0, T, n_head, ctx, 0, 0, 0};
     if (D == 128) {
-        launch_att<128>(a, stream);
+        launch_att<128>(a, (int64_t)batch * n_head, stream);
     } else {
-        launch_att<64>(a, stream);
+        launch_att<64>(a, (int64_t)batch * n_head, stream);
     }
     return check_launch("nb_attention_rows");
 }

@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "nativebit_amd.h"
 
 namespace nb {
@@ -181,7 +183,17 @@ int static_attention_scratch(hipStream_t stream, float** work, unsigned** done);
 int static_attention_max_heads();
 int64_t static_attention_scratch_bytes();
 
-// Batched-pass kernels (nb_rows.hip); arguments validated.
+// launch(first, count) over ranges of `heads` (the heads of every sequence)
+// whose blocks, `per_head` each of `threads`, keep a launch under 2^32
+// work-items, the most that one dimension of a grid takes.
+template <typename F>
+void for_head_ranges(int64_t heads, int64_t per_head, int threads, F&& launch) {
+    const int64_t most = std::max<int64_t>(0xffffffffLL / threads / per_head, 1);
+    for (int64_t h = 0; h < heads; h += most) launch((int)h, (int)std::min(most, heads - h));
+}
+
+// Batched-pass kernels (nb_rows.hip); arguments validated, batch * n_head
+// under 2^31.
 int launch_rmsnorm_rows(float* x, const float* add, const float* emb, const int32_t* tokens,
                         int vocab, const float* w, void* h, int h_dtype, int T, int C, float eps,
                         hipStream_t stream);

@@ -242,9 +242,10 @@ __global__ __launch_bounds__(64) void rope_kv_token_kernel(
 __global__ __launch_bounds__(kRopeThreads) void rope_kv_rows_kernel(
     const float* __restrict__ qkv, float* __restrict__ k_cache, float* __restrict__ v_cache,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t, int pos0, int T,
-    float* __restrict__ q_out, int n_head, int D, int ctx, int tiles) {
+    float* __restrict__ q_out, int n_head, int D, int ctx, int tiles, int head0) {
     __shared__ float ks[kRopeMaxD][kRT + 1];
-    const int bh = blockIdx.x / tiles, t0 = (blockIdx.x - bh * tiles) * kRT;
+    const int h0 = blockIdx.x / tiles, t0 = (blockIdx.x - h0 * tiles) * kRT;
+    const int bh = head0 + h0;
     const int b = bh / n_head, hd = bh - b * n_head;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int C = n_head * D, half = D / 2;
@@ -296,13 +297,13 @@ constexpr int kKPitch = kKT + 4;         // floats per LDS row of k (one head di
 __global__ __launch_bounds__(kAttThreads) void attention_rows_kernel(
     const float* __restrict__ q, const float* __restrict__ k_cache,
     const float* __restrict__ v_cache, int pos0, int T, void* __restrict__ out, int out_dtype,
-    int n_head, int D, int ctx) {
+    int n_head, int D, int ctx, int head0) {
     typedef __attribute__((ext_vector_type(4))) float f4;
     __shared__ __align__(16) float qs[kQB][kQPitch];
     __shared__ __align__(16) float ks[kRowsMaxD][kKPitch];   // keys transposed: [dim][position]
     __shared__ __align__(16) float vs[kKT][kQPitch];
     __shared__ __align__(16) float ps[kQB][kKPitch];
-    const int bh = blockIdx.x, t0 = blockIdx.y * kQB;
+    const int bh = head0 + blockIdx.x, t0 = blockIdx.y * kQB;
     const int b = bh / n_head, hd = bh - b * n_head;
     const int tid = threadIdx.x;
     const int C = n_head * D;
@@ -446,9 +447,11 @@ int launch_rope_kv_rows(const float* qkv, float* k_cache, float* v_cache, const 
         return check_launch("nb_rope_kv_rows");
     }
     const int tiles = (T + kRT - 1) / kRT;
-    hipLaunchKernelGGL(rope_kv_rows_kernel, dim3((unsigned)(batch * n_head * tiles)),
-                       dim3(kRopeThreads), 0, stream, qkv, k_cache, v_cache, cos_t, sin_t, pos0, T,
-                       q_out, n_head, D, ctx, tiles);
+    for_head_ranges(heads, tiles, kRopeThreads, [&](int head0, int count) {
+        hipLaunchKernelGGL(rope_kv_rows_kernel, dim3((unsigned)count * tiles), dim3(kRopeThreads), 0,
+                           stream, qkv, k_cache, v_cache, cos_t, sin_t, pos0, T, q_out, n_head, D,
+                           ctx, tiles, head0);
+    });
     return check_launch("nb_rope_kv_rows");
 }
 
@@ -467,9 +470,11 @@ int launch_attention_rows(const float* q, const float* k_cache, const float* v_c
         return launch_attention_mfma(q, k_cache, v_cache, pos0, T, out, out_dtype, batch, n_head, D,
                                      ctx, stream);
     }
-    hipLaunchKernelGGL(attention_rows_kernel, dim3(batch * n_head, (T + kQB - 1) / kQB),
-                       dim3(kAttThreads), 0, stream, q, k_cache, v_cache, pos0, T, out, out_dtype,
-                       n_head, D, ctx);
+    for_head_ranges((int64_t)batch * n_head, 1, kAttThreads, [&](int head0, int count) {
+        hipLaunchKernelGGL(attention_rows_kernel, dim3(count, (T + kQB - 1) / kQB),
+                           dim3(kAttThreads), 0, stream, q, k_cache, v_cache, pos0, T, out,
+                           out_dtype, n_head, D, ctx, head0);
+    });
     return check_launch("nb_attention_rows");
 }
 

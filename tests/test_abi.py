@@ -663,3 +663,23 @@ def test_prefill_best_entry_needs_its_own_workspace(name):
     assert call(name + "_best", None, best) == _lib.NB_EINVAL
     assert call(name + "_best", FAKE + 16, best) == _lib.NB_EALIGN
     assert getattr(lib, name + "_best_ws_bytes")(M, N, 100) == 0
+
+
+@pytest.mark.parametrize("call", ["rope", "attention"])
+def test_row_batches(call):
+    """Batches are refused only where their heads pass an int; an empty one
+    does nothing."""
+    lib = _lib.load()
+
+    def run(batch, n_head=20, T=1, ctx=64, D=128):
+        if call == "rope":
+            return lib.nb_rope_kv_batch(FAKE, FAKE, FAKE, FAKE, FAKE, 0, T, FAKE, batch, n_head, D,
+                                        ctx, None)
+        return lib.nb_attention_batch(FAKE, FAKE, FAKE, 0, T, FAKE, _lib.NB_F32, batch, n_head, D,
+                                      ctx, None)
+    assert run(-1) == _lib.NB_EINVAL
+    assert run(1 << 20, 1 << 11) == _lib.NB_EUNSUPPORTED
+    assert run(0) == _lib.NB_OK
+    assert run(4, T=0) == _lib.NB_OK
+    if not gpu_available():   # valid calls end at the missing device
+        assert run((1 << 20) - 1, 1 << 11, T=64) not in (_lib.NB_EINVAL, _lib.NB_EUNSUPPORTED)

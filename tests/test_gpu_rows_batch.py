@@ -64,6 +64,51 @@ def test_batch_equals_sequences(dev, B, H, D, ctx, pos0, T):
     assert (k[..., span] - rot).abs().max() <= 4 * 2.0 ** -24 * kk.abs().max()
 
 
+@pytest.mark.parametrize("kind,D,T,ctx,B", [
+    ("rope", 2, 33, 36, 8400),        # 2 workgroups a head: the second launch from head 8388607
+    ("attention", 2, 1, 4, 16800),    # the vector kernel: from head 16777215
+    ("attention", 64, 1, 4, 16800)])  # the MFMA kernel: from head 16777215
+def test_more_workgroups_than_a_launch_takes(dev, kind, D, T, ctx, B):
+    """2^24 workgroups of 256 threads are one launch too many (2^32
+    work-items): the call covers every head with several, as the sequences
+    around the seam, the first and the last ones show."""
+    H = 1000
+    need = 4 * B * H * D * (T * (4 if kind == "rope" else 2) + ctx * 2)
+    if torch.cuda.mem_get_info()[0] < 1.2 * need:
+        pytest.skip("not enough free memory")
+    print(f"[case] rows launches {kind} D={D} T={T} B={B} ({need >> 30} GiB)", flush=True)
+    lib, C = _lib.load(), H * D
+    cos, sin = (t.to(dev).contiguous() for t in precompute_rope(D, ctx))
+
+    def call(n, x, k, v):
+        out = torch.empty(n, T, C, device=dev)
+        if kind == "rope":
+            _lib.check(lib.nb_rope_kv_batch(P(x), P(k), P(v), P(cos), P(sin), 0, T, P(out), n, H, D,
+                                            ctx, stream()))
+            return out, k, v
+        _lib.check(lib.nb_attention_batch(P(x), P(k), P(v), 0, T, P(out), _lib.NB_F32, n, H, D, ctx,
+                                          stream()))
+        return (out,)
+
+    def caches(n):
+        if kind == "rope":
+            return torch.zeros(n, H, D, ctx, device=dev), torch.zeros(n, H, ctx, D, device=dev)
+        return k_all[:n], k_all[:n].view(n, H, ctx, D)   # (any numbers)
+
+    x = torch.empty(B, T, (3 if kind == "rope" else 1) * C, device=dev).normal_()
+    if kind == "attention":
+        k_all = torch.empty(B, H, D, ctx, device=dev).normal_()
+    got = call(B, x, *caches(B))
+    for b in {0, (2 ** 24 - 1) // (2 if kind == "rope" else 1) // H, B - 1}:
+        if kind == "rope":
+            one = call(1, x[b:b + 1].clone(), *caches(1))
+        else:
+            one = call(1, x[b:b + 1].clone(), k_all[b:b + 1].clone(),
+                       k_all[b:b + 1].clone().view(1, H, ctx, D))
+        assert all(torch.equal(g[b], o[0]) for g, o in zip(got, one))
+        assert one[0].abs().sum() > 0
+
+
 @pytest.mark.parametrize("D,ctx,pos0", [(32, 40, 20), (128, 40, 20), (128, 40, 36), (128, 41, 20)])
 def test_a_batch_is_one_launch(dev, D, ctx, pos0):
     """nb_rope_kv_batch and nb_attention_batch are one graph node each, on
