@@ -298,9 +298,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attention_mfma_kernel(AttArgs 
         float l = 0.f;
         f32x4_t v = {0.f, 0.f, 0.f, 0.f};
         for (int w = 0; w < kWaves; ++w) {
-            const float mw = om[w * 16 + qi];
-            if (mw == -INFINITY && ol[w * 16 + qi] == 0.f) continue;   // saw no key
-            const float f = __expf(mw - m);
+            // (a wave that saw no key, or only scores of -inf, has f = 0; its
+            // sums are zero, or NaN where such a key's value is not finite)
+            const float f = __expf(om[w * 16 + qi] - m);
             l += f * ol[w * 16 + qi];
             v += f * *reinterpret_cast<const f32x4_t*>(oo + (w * 16 + qi) * kPitch + d);
         }

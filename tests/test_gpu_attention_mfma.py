@@ -97,3 +97,24 @@ def test_nan_and_infinite_scores(dev):
     kc[0, 9, 70] = float("-inf")
     out = run(dev, q, kc, vc, pos0, H, D, ctx)
     assert (out - reference(q, kc, vc, pos0, H, D)).abs().max() <= 2e-5 * vc.abs().max()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_weight_zero_times_infinite_value(dev, D):
+    """A key that a query sees with a score of -inf has the weight 0, and 0
+    times an infinite value is NaN, also where its whole key tile (one wave's)
+    scores -inf; keys alone at -inf leave 0 / 0."""
+    H, ctx, pos0, T = 1, 256, 200, 3
+    q, kc, vc = inputs(H, D, ctx, T, 2)
+    q[:, 9] = 1.0
+    kc[0, 9, :64] = float("-inf")
+    vc[0, 10, 5] = float("inf")
+    out = run(dev, q, kc, vc, pos0, H, D, ctx)
+    assert out[:, 5].isnan().all()
+    clean = vc.clone()
+    clean[0, 10, 5] = 0.0
+    ref = reference(q, kc, clean, pos0, H, D)
+    rest = torch.arange(D) != 5
+    assert (out - ref)[:, rest].abs().max() <= 2e-5 * clean.abs().max()
+    kc[0, 9] = float("-inf")
+    assert run(dev, q, kc, clean, pos0, H, D, ctx).isnan().all()
