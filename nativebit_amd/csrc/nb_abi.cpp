@@ -778,10 +778,10 @@ int check_batch_size(const char* fn, int batch, int n_head) {
 int rope_kv(const char* fn, const float* qkv, float* k_cache, float* v_cache, const float* cos_t,
             const float* sin_t, int pos0, int T, float* q_out, int batch, int n_head, int head_dim,
             int ctx, void* stream) {
-    int st = check_rows_attention(fn, pos0, T, n_head, head_dim, ctx);
+    int st = check_batch_size(fn, batch, n_head);
+    if (st || batch == 0) return st;   // (no sequence: nothing to check or do)
+    st = check_rows_attention(fn, pos0, T, n_head, head_dim, ctx);
     if (st) return st;
-    st = check_batch_size(fn, batch, n_head);
-    if (st || batch == 0) return st;
     if (!qkv || !k_cache || !v_cache || !cos_t || !sin_t || !q_out) {
         return fail(NB_EINVAL, "%s: NULL pointer", fn);
     }
@@ -799,10 +799,10 @@ int rope_kv(const char* fn, const float* qkv, float* k_cache, float* v_cache, co
 int attention(const char* fn, const float* q, const float* k_cache, const float* v_cache, int pos0,
               int T, void* out, int out_dtype, int batch, int n_head, int head_dim, int ctx,
               void* stream) {
-    int st = check_rows_attention(fn, pos0, T, n_head, head_dim, ctx);
+    int st = check_batch_size(fn, batch, n_head);
+    if (st || batch == 0) return st;   // (no sequence: nothing to check or do)
+    st = check_rows_attention(fn, pos0, T, n_head, head_dim, ctx);
     if (st) return st;
-    st = check_batch_size(fn, batch, n_head);
-    if (st || batch == 0) return st;
     if (out_dtype != NB_F32 && out_dtype != NB_BF16) return fail(NB_EINVAL, "%s: out_dtype=%d", fn, out_dtype);
     if (!q || !k_cache || !v_cache || !out) return fail(NB_EINVAL, "%s: NULL pointer", fn);
     if (!aligned(q, 4) || !aligned(k_cache, 4) || !aligned(v_cache, 4) ||

@@ -679,7 +679,10 @@ def test_row_batches(call):
                                       ctx, None)
     assert run(-1) == _lib.NB_EINVAL
     assert run(1 << 20, 1 << 11) == _lib.NB_EUNSUPPORTED
-    assert run(0) == _lib.NB_OK
+    # (an empty batch also where a sequence would be refused: no positions in
+    # the cache, a head dim over 128)
+    assert run(0) == run(0, T=0, ctx=0) == run(0, D=256) == _lib.NB_OK
+    assert run(1, T=0, ctx=0) == _lib.NB_EINVAL and run(1, D=256) == _lib.NB_EUNSUPPORTED
     assert run(4, T=0) == _lib.NB_OK
     if not gpu_available():   # valid calls end at the missing device
         assert run((1 << 20) - 1, 1 << 11, T=64) not in (_lib.NB_EINVAL, _lib.NB_EUNSUPPORTED)
