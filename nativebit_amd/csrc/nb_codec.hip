@@ -849,7 +849,11 @@ int launch_dequant(const uint8_t* packed, const float* codebook, void* w,
             with_bits(bits, [&](auto B) {
                 constexpr int kB = decltype(B)::value;
                 if constexpr (kB >= 2 && kB <= 4) {
-                    if (n_entries == (1 << kB) && is_aligned(codebook, 16)) {
+                    // (one wave's worth to bf16 waits longer for its table than for
+                    // its lookups: 1024 weights of 16 entries 2.6 us against 2.3;
+                    // 4096 are even, 8192 2.9-3.0 against 3.1-3.8)
+                    if (n_entries == (1 << kB) && is_aligned(codebook, 16) &&
+                        !(bf16 && chunks <= 64)) {
                         auto tables = bf16 ? dequant_tables_kernel<kB, true>
                                            : dequant_tables_kernel<kB, false>;
                         hipLaunchKernelGGL(tables, dim3(grid_for(chunks)), dim3(kThreads), 0, stream,
