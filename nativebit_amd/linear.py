@@ -84,7 +84,15 @@ class PackedLinear(torch.nn.Module):
             # (.to(tl.float32), triton_kernel.py:46, 174-183)
             x_flat = x_flat.to(torch.float32)
         if M <= MAX_GEMV_ROWS:
-            y = ops.gemv(x_flat, self.packed_indices, self.codebook, N, K, bits=self.bits,
+            # the two attributes: nn.Module's own lookup takes 0.25 us each, so
+            # they come from where it finds them while they are plain buffers of
+            # this very class (not replaced by Parameters, parametrized, or
+            # properties of a subclass)
+            buffers = self._buffers
+            packed, codebook = buffers.get("packed_indices"), buffers.get("codebook")
+            if packed is None or codebook is None or type(self) is not PackedLinear:
+                packed, codebook = self.packed_indices, self.codebook
+            y = ops.gemv(x_flat, packed, codebook, N, K, bits=self.bits,
                          block_size=self.block_size, out_dtype=self.out_dtype)
         elif x_flat.dtype == torch.bfloat16 and self._standard():
             # the bf16 batched form (eval_ppl.py:149-174): the packed MFMA kernels

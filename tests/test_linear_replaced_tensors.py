@@ -36,6 +36,12 @@ def seen(monkeypatch):
     return calls
 
 
+class WithProperty(PackedLinear):
+    @property
+    def codebook(self):
+        return self._buffers["codebook"] + 7
+
+
 class Doubled(torch.nn.Module):
     def forward(self, t):
         return 2 * t
@@ -64,6 +70,11 @@ def test_replaced_tensors_are_used(seen, rows, dtype, n_entries):
     parametrize.register_parametrization(layer, "codebook", Doubled())
     layer(x)
     assert (seen.pop()[1] == 6).all()
+
+    layer = _layer(n_entries)
+    layer.__class__ = WithProperty
+    layer(x)
+    assert (seen.pop()[1] == 7).all()
 
     layer, other = _layer(n_entries), torch.full((N, n_entries), 5.0)
     torch.func.functional_call(layer, {"codebook": other}, (x,))
