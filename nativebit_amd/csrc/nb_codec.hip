@@ -806,8 +806,9 @@ int launch_block_codebooks(const float* w, int64_t total, int64_t num_blocks, in
     QuantileFractions qf;
     for (int e = 0; e < kCbMaxEntries; ++e) qf.q[e] = e < n_entries ? q[e] : 0.f;
     if (block_size <= 256) {
-        // 6912 x 2560, 8 entries: 98 us with one block a wave sorted by
-        // ds_bpermute shuffles, 31 us with four (70.8 MB read: 2.4 TB/s)
+        // 6912 x 2560, 8 entries, cold weights: 90 us with one block a wave
+        // sorted by ds_bpermute shuffles, 28 us with four (70.8 MB read: 2.5
+        // TB/s)
         const int64_t want = (num_blocks + kThreads / 16 - 1) / (kThreads / 16);
         const int64_t cap = (int64_t)device_cu_count() * 8;
         const int grid = (int)(want < cap ? want : cap);

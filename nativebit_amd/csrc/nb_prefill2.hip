@@ -207,9 +207,9 @@ struct WRegs {
 // rounded to bf16).  The fragments of a step then feed three MFMAs instead of
 // two, so this form reads less LDS per MFMA than the bf16 one.  Measured
 // against three passes of the bf16 kernel that added to y (and a residual
-// codebook made per call): 7680 x 2560 at M = 128 / 500 / 2048 34 / 71 / 221 us
-// (72 / 129 / 286), 2560 x 6912 34 / 68 / 227 us (78 / 145 / 313), the same
-// 4.3e-6 from fp64.
+// codebook made per call), with the fastest plans: 7680 x 2560 at M = 128 / 500
+// / 2048 36 / 74 / 232 us (73 / 127 / 298), 2560 x 6912 34 / 70 / 234 us (74 /
+// 144 / 308); 4.301e-6 from fp64 (4.295e-6: the three products share a sum).
 template <int BM, int BN, int WAVES, bool kSplit>
 __global__ __launch_bounds__(64 * WAVES) void prefill2_kernel(Prefill2Args a) {
     constexpr int kThreads = 64 * WAVES;
