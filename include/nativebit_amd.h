@@ -555,7 +555,8 @@ int nb_attention_rows(const float* q, const float* k_cache, const float* v_cache
                       void* out, int out_dtype, int n_head, int head_dim, int ctx, void* stream);
 /*
  * nb_rope_kv_rows and nb_attention_rows for `batch` sequences of T tokens at
- * the same positions in one launch: qkv, q_out, q and out hold the
+ * the same positions in one launch (several where it would pass 2^32
+ * work-items; nothing for an empty batch): qkv, q_out, q and out hold the
  * sequences' rows one after the other, the caches [batch][n_head][...].
  * Replaces: the same lines of CausalAttention.forward over the batch.
  */
